@@ -122,9 +122,9 @@ int eg_create(int device, eg_context** out_ctx) {
       ctx->attention_split_fill = (uint32_t)f;
     }
   }
-  if (const char* g = std::getenv("EG_PREFILL_GROUPS")) {
-    const int v = std::atoi(g);
-    if (v == 1 || v == 2 || v == 4) ctx->prefill_groups = v;
+  if (const char* g = std::getenv("EG_PREFILL_TILE")) {
+    int* t = ctx->gemm_tile;
+    if (std::sscanf(g, "%d,%d,%d,%d,%d", &t[0], &t[1], &t[2], &t[3], &t[4]) < 4) std::memset(t, 0, sizeof(ctx->gemm_tile));
   }
   err = hipMalloc(&ctx->workspace, eg::kWorkspaceBytes);
   if (err != hipSuccess) {
@@ -157,6 +157,8 @@ int eg_destroy(eg_context* ctx) {
   if (!ctx) return EG_OK;
   hipSetDevice(ctx->device);
   hipStreamSynchronize(ctx->own_stream);
+  if (ctx->rows_done) (void)hipEventDestroy(ctx->rows_done);
+  if (ctx->rows) (void)hipFree(ctx->rows);
   if (ctx->workspace) hipFree(ctx->workspace);
   hipStreamDestroy(ctx->own_stream);
   delete ctx;

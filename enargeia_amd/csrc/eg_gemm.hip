@@ -1,88 +1,39 @@
 // matmul_q4_prefill (matmul_q4_prefill.wgsl:77-162) on the matrix cores:
 //   out[r*out_stride + col + out_offset] = sum_k x[r,k] * W[col,k] (+ bias[col])
 //
-// The prefill chunk (M = 128-256 queries) is the one dense contraction on the path. Each
-// workgroup owns a 64 x 64 output tile and a slice of K; its 4 waves each own 32 x 32 = 2 x 2
-// tiles of v_mfma_f32_16x16x32_bf16. K is staged 64 at a time through LDS:
-//   * x (f32) is rounded to bf16 (round-to-nearest-even) on the way into LDS;
-//   * W is dequantized while staging, as the reference's prefill kernel does: 16 int4 codes
-//     (8 bytes, one scale and zero-point) per thread, dequantized in f32, then bf16 - so the
-//     codes cross HBM as int4 and each weight is unpacked once per tile, not once per MFMA
-//     that reads it.
-// The loop is latency-bound at these sizes (a few MFMAs per staged block), so:
-//   * global loads run two blocks ahead of the LDS staging, in three register stages;
-//   * K is split over grid.z when the tile grid alone would leave the device idle (the down
-//     projection has 4 x 14 tiles at M = 256): each split writes f32 partials into the context's
-//     workspace and a second launch sums the splits in index order, plus the bias - the result
-//     does not depend on how the work was scheduled.
-// Rows are padded by 16 bytes in LDS so the 16 lanes that read one column of A (or B) hit
-// different banks. Accumulation is f32 inside the MFMA.
-// Layouts the chunked staging cannot take (K or block size not a multiple of 32 codes, a block
-// size that is not a power of two, int8 codes, unaligned streams, K not a multiple of 4) stage
-// element by element with the reference's indexing.
+// The prompt's projections are the dense contraction on the path. This file holds the host side:
+// the checks, the choice of a tile for a shape (tile_for) and the launches. The kernel is
+// gemm_kernel (eg_gemm_kernel.hpp), instantiated in eg_gemm_{bf16,f32,norm,pair,rope}.hip.
+// Layouts it does not take (K or the block size not a multiple of 16 or 32 codes, a block size
+// that is not a power of two, unaligned streams) stage both operands element by element with the
+// reference's indexing (element_kernel below).
 #include <algorithm>
 
-#include "eg_internal.hpp"
+#include "eg_gemm_kernel.hpp"
 
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+using namespace eg_gemm;
+
+// ---- the element-by-element kernel ------------------------------------------------------------
 
 constexpr int kTile = 64;   // M and N tile
 constexpr int kBK = 64;     // K staged per iteration
 constexpr int kPad = 8;     // bf16 elements of padding per LDS row
 constexpr int kLds = kBK + kPad;
-constexpr int kStages = 3;  // register stages of the chunked staging pipeline
 
-// One matrix of a launch: its streams, outputs and the end of its range of 64-column tiles along
-// grid.x. A multi-matrix launch holds several that share x, M, K, the quant block size and the
-// encoding; the usual launch holds one.
-struct PrefillMat {
+struct ElementArgs {
+  const float* x;
   const uint32_t* packed;
   const float* scales;
   const uint32_t* zeros;
   const float* bias;
-  const float* residual;  // nullable: out = acc + bias + residual[r * out_stride + col + out_offset]
+  const float* residual;
   float* out;
-  uint32_t n, out_stride, out_offset, tiles_end;
-};
-constexpr uint32_t kMaxSegs = 3;
-
-struct PrefillArgs {
-  const float* x;
   float* partials;  // split-K: [splits][m][n] f32; NULL when grid.z == 1
-  uint32_t m, k, block_size, blocks_per_row, k_per_split;
+  uint32_t m, n, k, block_size, blocks_per_row, k_per_split, out_stride, out_offset;
   int bits;
-  uint32_t block_shift;  // log2(block_size) (the chunked staging takes power-of-two blocks)
-  uint32_t nmats;        // matrices in mats (> 1: no K split)
-  const float* norm;     // NORM launches: x is RMS-normalised per row with these weights (no K split)
-  float eps;
-  // ROPE launches (q | k | v, 64-column tiles = heads): q rows rotated and scaled by 1/8 into
-  // q_rope [row][q heads][64], k rows rotated and v rows as they are into the f16 caches at
-  // positions rope_pos0 + row ([pos][kv_heads][64]); rope = the cos/sin table [pos][32]
-  const double2* rope;
-  float* q_rope;
-  uint16_t* k_cache;
-  uint16_t* v_cache;
-  uint32_t rope_pos0, q_heads, kv_heads;
-  uint32_t out_bf16;  // PAIR launches: SiLU(g) * u stored as bf16 (the next GEMM's x, bit-for-bit
-                      // what its staging would round it to)
-  uint32_t xcd_rows;  // grid.y a multiple of 8, grid.z 1: tiles mapped so that each XCD runs whole
-                      // row tiles (below)
-  PrefillMat mats[kMaxSegs];
 };
-
-// The matrix that owns tile column `tx` and the first tile column of its range. The matrix is
-// read in place from the kernel arguments (the arguments are never written: a written copy with
-// an indexed array member would be kept in scratch memory).
-__device__ __forceinline__ uint32_t select_matrix(const PrefillArgs& a, uint32_t tx) {
-  uint32_t s = 0;
-#pragma unroll
-  for (uint32_t i = 0; i + 1 < kMaxSegs; i++)
-    if (i + 1 < a.nmats && tx >= a.mats[i].tiles_end) s = i + 1;
-  return s;
-}
 
 __device__ __forceinline__ uint16_t bf16_bits(float v) {
   uint32_t u = __float_as_uint(v);
@@ -91,147 +42,9 @@ __device__ __forceinline__ uint16_t bf16_bits(float v) {
   return (uint16_t)(u >> 16);
 }
 
-using egd::pack_bf16;
-
-// One 64 x 64 block of x and of W held in registers between its global loads and its LDS
-// stores (chunked layout): x as 4 float4 per thread; W as 16 codes (8 bytes) per thread - row
-// tid / 4, codes 16 * (tid % 4) .. +16 of the block - with their block's scale and zero-point.
-struct Staged {
-  float4 x[4];
-  float4 g;  // NORM: the norm weights of the 4 x columns
-  uint2 q;
-  float s;
-  float z;
-};
-
-// The four streams as buffer resources: an out-of-range offset reads zeros without touching
-// memory, so a block's edge needs no branch (a branch around a load makes the compiler wait
-// for it on the spot, which would serialize the stages).
-struct Streams {
-  __amdgpu_buffer_rsrc_t x, w, s, z, g;
-};
-constexpr uint32_t kOutside = 0x80000000u;  // an offset past every stream (streams < 2 GiB here)
-
-// This thread's part of every staged block, fixed for the launch: its 4 x vectors (rows
-// m0 + tid/16 + 16i, columns 4 * (tid % 16) of the block) and its 16 codes (row n0 + tid/4,
-// columns 16 * (tid % 4) of the block). A block's loads are then these bases plus the block's
-// column, with no per-block multiplies.
-struct StageBase {
-  uint32_t x[4];    // byte offset of row r_i, column c (block 0), or kOutside when the row is outside
-  uint32_t xc;      // column of the x vectors within a block
-  uint32_t w;       // byte offset of the codes (block 0), or kOutside when the row is outside
-  uint32_t kc;      // column of the codes within a block
-  uint32_t sblk;    // the row's first quant block index
-};
-
-template <bool XB16>
-__device__ __forceinline__ StageBase stage_base(const PrefillArgs& a, const PrefillMat& w, uint32_t m0, uint32_t n0) {
-  const uint32_t tid = threadIdx.x & 255u;  // the thread within its group of 4 waves
-  StageBase b;
-  b.xc = (tid & 15u) * 4u;
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const uint32_t row = m0 + (tid >> 4) + 16u * i;
-    b.x[i] = row < a.m ? (row * a.k + b.xc) * (XB16 ? 2u : 4u) : kOutside;
-  }
-  const uint32_t nrow = n0 + (tid >> 2);
-  b.kc = 16u * (tid & 3u);
-  b.w = nrow < w.n ? (nrow * a.k + b.kc) / 2u : kOutside;
-  b.sblk = nrow * a.blocks_per_row;
-  return b;
-}
-
-template <int ENC, bool NORM, bool XB16>
-__device__ __forceinline__ void load_block(const PrefillArgs& a, const Streams& r, const StageBase& b, uint32_t k0,
-                                           Staged& st) {
-  const bool xin = k0 + b.xc < a.k;
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    if (XB16) {  // 4 bf16 values, kept as their bits in x and y
-      const uint64_t v = egd::load_b64(r.x, xin && b.x[i] != kOutside ? b.x[i] + k0 * 2u : kOutside);
-      st.x[i] = make_float4(__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32)), 0.f, 0.f);
-    } else {
-      const egd::u32x4 v = egd::load_b128(r.x, xin && b.x[i] != kOutside ? b.x[i] + k0 * 4u : kOutside);
-      st.x[i] = make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
-    }
-  }
-  if (NORM) {
-    const egd::u32x4 v = egd::load_b128(r.g, xin ? (k0 + b.xc) * 4u : kOutside);
-    st.g = make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
-  }
-  const bool in = b.w != kOutside && k0 + b.kc < a.k;
-  const uint32_t blk = b.sblk + ((k0 + b.kc) >> a.block_shift);
-  const uint64_t codes = egd::load_b64(r.w, in ? b.w + k0 / 2u : kOutside);
-  st.q = make_uint2((uint32_t)codes, (uint32_t)(codes >> 32));
-  st.s = egd::load_f32(r.s, in ? blk * 4u : kOutside);
-  if (ENC == EG_ENC_OFFSET_ZEROS) {
-    const uint32_t zw = egd::load_b32(r.z, in ? (blk / 8u) * 4u : kOutside);
-    st.z = (float)((zw >> (4 * (blk % 8))) & 0xFu);
-  } else {
-    st.z = 8.f;
-  }
-}
-
-template <int ENC, bool NORM, bool XB16>
-__device__ __forceinline__ void store_block(const Staged& st, uint16_t (*As)[kLds], uint16_t (*Bs)[kLds]) {
-  const uint32_t tid = threadIdx.x & 255u;
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const uint32_t idx = tid + i * 256u;
-    const uint32_t r = idx >> 4, c = (idx & 15u) * 4u;
-    if (XB16) {
-      *reinterpret_cast<uint2*>(&As[r][c]) = make_uint2(__float_as_uint(st.x[i].x), __float_as_uint(st.x[i].y));
-      continue;
-    }
-    // NORM: x times its column's norm weight here, the row's 1 / rms in the epilogue
-    const float4 v = NORM ? make_float4(st.x[i].x * st.g.x, st.x[i].y * st.g.y, st.x[i].z * st.g.z, st.x[i].w * st.g.w)
-                          : st.x[i];
-    *reinterpret_cast<uint2*>(&As[r][c]) = make_uint2(pack_bf16(v.x, v.y), pack_bf16(v.z, v.w));
-  }
-  // (code - zero) * scale in f32, exactly the reference's dequantElement, then bf16. Each word's
-  // low and high nibbles are masked in place (the high ones stay 16x, their scale is divided
-  // by 16: exact) and each byte converts straight to f32. Two's-complement codes are flipped
-  // to offset binary c = q + 8 in the same mask, and c * s - 8 * s is one fused multiply-add:
-  // the product is exact inside it and 8 * s is exact, so the single rounding is that of
-  // (c - 8) * s. Offset-binary codes keep the subtraction: (c - z) * s.
-  const uint32_t d[2] = {st.q.x, st.q.y};
-  const float s16 = st.s * 0.0625f;
-  uint32_t packed[8];
-#pragma unroll
-  for (int w = 0; w < 2; w++) {
-    uint32_t lo, hi;
-    if (ENC == EG_ENC_SIGNED) {
-      lo = (d[w] & 0x0F0F0F0Fu) ^ 0x08080808u;
-      hi = (d[w] & 0xF0F0F0F0u) ^ 0x80808080u;
-    } else {
-      lo = egd::and_opaque(d[w], 0x0F0F0F0Fu);
-      hi = egd::and_opaque(d[w], 0xF0F0F0F0u);
-    }
-    float v[8];
-    const float cl[4] = {egd::ub0(lo), egd::ub1(lo), egd::ub2(lo), egd::ub3(lo)};
-    const float ch[4] = {egd::ub0(hi), egd::ub1(hi), egd::ub2(hi), egd::ub3(hi)};
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      if (ENC == EG_ENC_SIGNED) {
-        const float off = -8.f * st.s;
-        v[2 * j] = fmaf(cl[j], st.s, off);
-        v[2 * j + 1] = fmaf(ch[j], s16, off);
-      } else {
-        v[2 * j] = (cl[j] - st.z) * st.s;
-        v[2 * j + 1] = (ch[j] - 16.f * st.z) * s16;
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < 8; e += 2) packed[(w * 8 + e) / 2] = pack_bf16(v[e], v[e + 1]);
-  }
-  uint4* dst = reinterpret_cast<uint4*>(&Bs[tid >> 2][16u * (tid & 3u)]);
-  dst[0] = make_uint4(packed[0], packed[1], packed[2], packed[3]);
-  dst[1] = make_uint4(packed[4], packed[5], packed[6], packed[7]);
-}
-
-// Element-by-element staging for the layouts the chunked path does not take.
+// One 64 x 64 block of x and of W into LDS.
 template <int ENC>
-__device__ void stage_elements(const PrefillArgs& a, const PrefillMat& w, uint32_t m0, uint32_t n0, uint32_t k0,
+__device__ void stage_elements(const ElementArgs& a, uint32_t m0, uint32_t n0, uint32_t k0,
                                uint16_t (*As)[kLds], uint16_t (*Bs)[kLds]) {
   const uint32_t tid = threadIdx.x & 255u;
   const uint32_t per_word = 32u / (uint32_t)a.bits, mask = (1u << a.bits) - 1u;
@@ -247,311 +60,91 @@ __device__ void stage_elements(const PrefillArgs& a, const PrefillMat& w, uint32
     const uint32_t r = e / kBK, c = e % kBK;
     const uint32_t nrow = n0 + r, kk = k0 + c;
     float v = 0.f;
-    if (nrow < w.n && kk < a.k) {
+    if (nrow < a.n && kk < a.k) {
       const size_t flat = (size_t)nrow * a.k + kk;
-      uint32_t code = (w.packed[flat / per_word] >> (a.bits * (flat % per_word))) & mask;
+      uint32_t code = (a.packed[flat / per_word] >> (a.bits * (flat % per_word))) & mask;
       const uint32_t blk = nrow * a.blocks_per_row + kk / a.block_size;
       int32_t z;
       if (ENC == EG_ENC_OFFSET_ZEROS) {
-        z = (int32_t)((w.zeros[blk / per_word] >> (a.bits * (blk % per_word))) & mask);
+        z = (int32_t)((a.zeros[blk / per_word] >> (a.bits * (blk % per_word))) & mask);
       } else {
         code ^= 1u << (a.bits - 1);
         z = 1 << (a.bits - 1);
       }
-      v = (float)((int32_t)code - z) * w.scales[blk];
+      v = (float)((int32_t)code - z) * a.scales[blk];
     }
     Bs[r][c] = bf16_bits(v);
   }
 }
 
-// v rounded to bf16 as pack_bf16 rounds it (round to nearest even).
-__device__ __forceinline__ uint16_t bf16_of(float v) { return (uint16_t)(pack_bf16(v, 0.f) & 0xFFFFu); }
-
-// SiLU(g) * u with SiLU(g) = g / (1 + e^-g), the prompt chain's silu_mul_rows formula.
-__device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.0f + expf(-g)) * u; }
-
-// KG groups of 4 waves share a workgroup and a tile: group g stages and multiplies the 64-deep
-// blocks g, g + KG, ... of the workgroup's K range into its own accumulators (its own LDS
-// buffers; one barrier pair per KG blocks), and the groups' sums are added in group order at the
-// end. With one workgroup per CU (the tile grids here hold ~1 per CU) a single group leaves
-// every SIMD one wave, so each block's staging, LDS round trip, barriers and MFMAs run back to
-// back; KG groups put KG waves on each SIMD and cut the serial chain by KG.
-//
-// PAIR (the gate|up SwiGLU pair, chunked staging only): tile column t holds rows 32t .. 32t+31 of
-// mats[0] (gate) in its first 32 columns and the same rows of mats[1] (up) in the last 32 - waves
-// 0-1 of a group stage gate rows, waves 2-3 up rows - and the epilogue stores SiLU(gate) * up for
-// the 32 columns into mats[0].out.
-//
-// NORM (chunked staging, no K split): x is a residual row, RMS-normalised on the way in - each
-// staged x value times its column's norm weight before the bf16 rounding, each thread summing
-// the squares of the x it stages; the rows' sums meet in LDS after the K loop and the epilogue
-// scales each output row by 1 / sqrt(sum / K + eps) (rmsnorm_rows' formula, with the row's
-// scale applied after the products instead of before them).
-//
-// ROPE (chunked staging; mats = q, k, v with head_dim 64, so a tile is one head): the epilogue
-// takes each row's (e, e + 32) pairs from the LDS sums, adds the biases, rotates them in double
-// precision with the table's cos/sin of the row's position - rope_append's arithmetic - and
-// stores q * RoPE / 8 in f32 and k, v in f16 into the caches.
-//
-// XB16 (chunked staging, no NORM): x holds bf16 values (a producer stored them rounded as the
-// staging would), staged as they are.
-//
-// S: register stages of the chunked staging (blocks in flight per group: S - 1). Four groups fit
-// four waves per SIMD only within 128 VGPRs: they keep one block in flight. Measured on the
-// config-3 shapes, deeper staging does not pay: one group at S = 5 runs as S = 3, at S = 8 (one
-// wave per SIMD) 18.5 -> 27.4 us for gate M = 256; two groups at S = 4 and four at S = 3 are
-// slower than their defaults.
-template <int ENC, bool CHUNKED, int KG, bool PAIR = false, bool NORM = false, bool ROPE = false, bool XB16 = false,
-          int S = (KG >= 4 ? 2 : kStages)>
-__global__ __launch_bounds__(256 * KG) void prefill_kernel(PrefillArgs a) {
-  // No contraction of separate operations into fused multiply-adds (the explicit fmaf calls stay):
-  // every epilogue then rounds the row's norm scale and the bias addition on their own, so the
-  // launches that fold different work into their epilogues give the same values.
+// A workgroup owns a 64 x 64 output tile and a slice of K, KG groups of 4 waves the 64-deep blocks
+// g, g + KG, ... of it (each wave 32 x 32 of the tile); the groups' sums meet in LDS and are added
+// in group order.
+template <int ENC, int KG>
+__global__ __launch_bounds__(256 * KG) void element_kernel(ElementArgs a) {
 #pragma clang fp contract(off)
-  // staging buffers of every group; after the K loop they hold the groups' f32 sums
   constexpr uint32_t kStageBytes = 2u * kTile * kLds * 2u;  // As + Bs of one group
   static_assert(kStageBytes >= kTile * kTile * 4u, "a group's buffers hold its 64 x 64 f32 sums");
   __shared__ __attribute__((aligned(16))) uint8_t lds[KG * kStageBytes];
-  __shared__ float row_ss[NORM ? KG : 1][kTile];  // NORM: each group's sums of squares per row
   const uint32_t group = threadIdx.x >> 8;
   uint16_t(*As)[kLds] = reinterpret_cast<uint16_t(*)[kLds]>(lds + group * kStageBytes);
   uint16_t(*Bs)[kLds] = reinterpret_cast<uint16_t(*)[kLds]>(lds + group * kStageBytes + kTile * kLds * 2u);
   const uint32_t tid = threadIdx.x & 255u, wave = tid >> 6, lane = tid & 63u;
-  // The tile (tx, ty). Workgroups are dispatched to the 8 XCDs in turn (workgroup L of the grid
-  // on XCD L % 8), each with its own L2. With xcd_rows the workgroups of one XCD take whole row
-  // tiles (row tiles k, k + 8, ... on XCD k, every column tile of each), so a row tile's x is
-  // fetched into one L2 instead of up to eight; otherwise the grid's own order.
-  uint32_t tx = blockIdx.x, ty = blockIdx.y;
-  if (a.xcd_rows) {
-    const uint32_t L = blockIdx.x + gridDim.x * blockIdx.y, k = L % 8u, j = L / 8u;
-    ty = k + 8u * (j / gridDim.x);
-    tx = j % gridDim.x;
-  }
-  // the matrix whose rows this thread stages (wave-uniform), and the tile's first row of it
-  const uint32_t half = PAIR ? __builtin_amdgcn_readfirstlane(wave >> 1) : 0u;
-  const PrefillMat& w = a.mats[PAIR ? half : select_matrix(a, tx)];
-  const uint32_t m0 = ty * kTile;
-  const uint32_t n0 = PAIR ? 32u * tx - 32u * half : (tx - (w.tiles_end - ((w.n + kTile - 1) / kTile))) * kTile;
+  const uint32_t m0 = blockIdx.y * kTile, n0 = blockIdx.x * kTile;
   const uint32_t wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
   const uint32_t kbeg = blockIdx.z * a.k_per_split, kend = min(a.k, kbeg + a.k_per_split);
-
   f32x4 acc[2][2];
 #pragma unroll
   for (int i = 0; i < 2; i++)
 #pragma unroll
     for (int j = 0; j < 2; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  auto mfma_block = [&]() {
-#pragma unroll
-    for (int ks = 0; ks < kBK / 32; ks++) {
-      const uint32_t kofs = ks * 32 + 8 * (lane >> 4);
-      bf16x8 af[2], bfr[2];
-#pragma unroll
-      for (int i = 0; i < 2; i++) {
-        const uint4 ua = *reinterpret_cast<const uint4*>(&As[wm + i * 16 + (lane & 15)][kofs]);
-        af[i] = __builtin_bit_cast(bf16x8, ua);
-        const uint4 ub = *reinterpret_cast<const uint4*>(&Bs[wn + i * 16 + (lane & 15)][kofs]);
-        bfr[i] = __builtin_bit_cast(bf16x8, ub);
-      }
-#pragma unroll
-      for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bfr[j], acc[i][j], 0, 0, 0);
-    }
-  };
-
-  const uint32_t nblk = (kend - kbeg + kBK - 1) / kBK;
-  // this group's blocks: group + KG * i for i < iters (the last ones past nblk are skipped; the
-  // groups run the same number of iterations so the barriers match)
-  const uint32_t iters = (nblk + KG - 1) / KG;
-  auto block_of = [&](uint32_t i) { return group + KG * i; };
-  if (CHUNKED) {
-    // kStages register stages: block b lives in stage b % kStages and is stored to LDS while
-    // blocks b+1 .. b+kStages-1 are in flight (an iteration is ~0.3 us of staging and MFMAs;
-    // HBM latency is several of those). The steady-state loop covers whole groups of kStages
-    // blocks with no branch at all - loads unconditional, clamped to the last block - so the
-    // compiler's wait before each store counts exactly the loads issued after that stage's; the
-    // remaining blocks are already in flight and drain in a loop that issues no loads.
-    const Streams rs{egd::buffer(a.x, a.m * a.k * (XB16 ? 2u : 4u)), egd::buffer(w.packed, w.n * a.k / 2u),
-                     egd::buffer(w.scales, w.n * a.blocks_per_row * 4u),
-                     egd::buffer(w.zeros, ((w.n * a.blocks_per_row + 7u) / 8u) * 4u),
-                     egd::buffer(NORM ? a.norm : nullptr, NORM ? a.k * 4u : 0u)};
-    const StageBase sb = stage_base<XB16>(a, w, m0, n0);
-    Staged st[S];
-    float ss[4] = {0.f, 0.f, 0.f, 0.f};  // NORM: squares of this thread's x, rows tid / 16 + 16 i
-    auto square = [&](const Staged& v) {
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        ss[i] = fmaf(v.x[i].x, v.x[i].x, ss[i]);
-        ss[i] = fmaf(v.x[i].y, v.x[i].y, ss[i]);
-        ss[i] = fmaf(v.x[i].z, v.x[i].z, ss[i]);
-        ss[i] = fmaf(v.x[i].w, v.x[i].w, ss[i]);
-      }
-    };
-#pragma unroll
-    for (int u = 0; u + 1 < S; u++)
-      load_block<ENC, NORM, XB16>(a, rs, sb, kbeg + min(block_of((uint32_t)u), nblk - 1) * kBK, st[u]);
-    const uint32_t full = iters / S;
-    for (uint32_t g = 0; g < full; g++) {
-#pragma unroll
-      for (int u = 0; u < S; u++) {
-        const uint32_t it = g * S + u;
-        store_block<ENC, NORM, XB16>(st[u], As, Bs);
-        if (NORM && block_of(it) < nblk) square(st[u]);
-        __syncthreads();
-        load_block<ENC, NORM, XB16>(a, rs, sb, kbeg + min(block_of(it + S - 1), nblk - 1) * kBK, st[(u + S - 1) % S]);
-        if (block_of(it) < nblk) mfma_block();
-        __syncthreads();
-      }
-    }
-    const uint32_t rest = iters - full * S;
-#pragma unroll
-    for (int u = 0; u + 1 < S; u++) {
-      if ((uint32_t)u < rest) {
-        store_block<ENC, NORM, XB16>(st[u], As, Bs);
-        if (NORM && block_of(full * S + u) < nblk) square(st[u]);
-        __syncthreads();
-        if (block_of(full * S + u) < nblk) mfma_block();
-        __syncthreads();
-      }
-    }
-    if (NORM) {
-      // the 16 threads of a row group (lanes 16 q .. 16 q + 15 of a wave) hold the row's columns
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int off = 1; off < 16; off <<= 1) ss[i] += __shfl_xor(ss[i], off, 64);
-      if ((tid & 15u) == 0)
-#pragma unroll
-        for (int i = 0; i < 4; i++) row_ss[NORM ? group : 0][(tid >> 4) + 16 * i] = ss[i];
-      __syncthreads();
-    }
-  } else {
-    for (uint32_t it = 0; it < iters; it++) {
-      const uint32_t blk = min(block_of(it), nblk - 1);
-      stage_elements<ENC>(a, w, m0, n0, kbeg + blk * kBK, As, Bs);
-      __syncthreads();
-      if (block_of(it) < nblk) mfma_block();
-      __syncthreads();
-    }
-  }
-  // NORM: 1 / rms of tile row r, the groups' sums of squares added in group order
-  auto inv_rms = [&](uint32_t r) {
-    float t = row_ss[0][r];
-#pragma unroll
-    for (int g = 1; g < (NORM ? KG : 1); g++) t += row_ss[NORM ? g : 0][r];
-    return 1.0f / sqrtf(t / (float)a.k + a.eps);
-  };
-  if (KG > 1 || PAIR || ROPE) {
-    // every group's sums into its own buffers (the last barrier above ended the staging), then
-    // the groups added in order by the thread that stores the element
-    float* sums = reinterpret_cast<float*>(lds + group * kStageBytes);
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int j = 0; j < 2; j++)
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-          sums[(wm + i * 16 + 4 * (lane >> 4) + e) * kTile + wn + j * 16 + (lane & 15)] = acc[i][j][e];
+  const uint32_t nblk = (kend - kbeg + kBK - 1) / kBK, iters = (nblk + KG - 1) / KG;
+  for (uint32_t it = 0; it < iters; it++) {
+    const uint32_t blk = group + KG * it;
+    stage_elements<ENC>(a, m0, n0, kbeg + min(blk, nblk - 1) * kBK, As, Bs);
     __syncthreads();
-    if (ROPE) {
-      const uint32_t s = select_matrix(a, tx), hd = n0 / kTile;
-      auto sum = [&](uint32_t r, uint32_t c) {
-        float v = reinterpret_cast<const float*>(lds)[r * kTile + c];
+    if (blk < nblk) {
 #pragma unroll
-        for (int k = 1; k < KG; k++) v += reinterpret_cast<const float*>(lds + k * kStageBytes)[r * kTile + c];
-        if (NORM) v *= inv_rms(r);
-        return v + (w.bias ? w.bias[n0 + c] : 0.f) + 0.f;
-      };
-      if (s == 2) {  // v: the rows as they are, f16
-        for (uint32_t idx = threadIdx.x; idx < kTile * kTile; idx += 256u * KG) {
-          const uint32_t r = idx / kTile, c = idx % kTile, row = m0 + r;
-          if (row >= a.m) continue;
-          a.v_cache[((size_t)(a.rope_pos0 + row) * a.kv_heads + hd) * kTile + c] = egd::float_to_half(sum(r, c));
-        }
-        return;
-      }
-      for (uint32_t idx = threadIdx.x; idx < kTile * 32u; idx += 256u * KG) {
-        const uint32_t r = idx / 32u, e = idx % 32u, row = m0 + r;
-        if (row >= a.m) continue;
-        const double2 cs = a.rope[(size_t)(a.rope_pos0 + row) * 32u + e];
-        const float2 rr = egd::rotate(sum(r, e), sum(r, e + 32u), cs);
-        const float r0 = rr.x, r1 = rr.y;
-        if (s == 0) {
-          float* dst = a.q_rope + ((size_t)row * a.q_heads + hd) * kTile;
-          dst[e] = r0 * 0.125f;
-          dst[e + 32u] = r1 * 0.125f;
-        } else {
-          uint16_t* dst = a.k_cache + ((size_t)(a.rope_pos0 + row) * a.kv_heads + hd) * kTile;
-          dst[e] = egd::float_to_half(r0);
-          dst[e + 32u] = egd::float_to_half(r1);
-        }
-      }
-      return;
-    }
-    if (PAIR) {
-      const PrefillMat& g = a.mats[0];
-      const PrefillMat& u = a.mats[1];
-      for (uint32_t idx = threadIdx.x; idx < kTile * 32u; idx += 256u * KG) {
-        const uint32_t r = idx / 32u, c = idx % 32u, row = m0 + r, col = 32u * tx + c;
-        if (row >= a.m || col >= g.n) continue;
-        float gv = reinterpret_cast<const float*>(lds)[r * kTile + c];
-        float uv = reinterpret_cast<const float*>(lds)[r * kTile + c + 32u];
+      for (int ks = 0; ks < kBK / 32; ks++) {
+        const uint32_t kofs = ks * 32 + 8 * (lane >> 4);
+        bf16x8 af[2], bfr[2];
 #pragma unroll
-        for (int k = 1; k < KG; k++) {
-          gv += reinterpret_cast<const float*>(lds + k * kStageBytes)[r * kTile + c];
-          uv += reinterpret_cast<const float*>(lds + k * kStageBytes)[r * kTile + c + 32u];
+        for (int i = 0; i < 2; i++) {
+          af[i] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&As[wm + i * 16 + (lane & 15)][kofs]));
+          bfr[i] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&Bs[wn + i * 16 + (lane & 15)][kofs]));
         }
-        if (NORM) {
-          const float inv = inv_rms(r);
-          gv *= inv;
-          uv *= inv;
-        }
-        gv = gv + (g.bias ? g.bias[col] : 0.f) + 0.f;
-        uv = uv + (u.bias ? u.bias[col] : 0.f) + 0.f;
-        const size_t o = (size_t)row * g.out_stride + col + g.out_offset;
-        if (a.out_bf16) reinterpret_cast<uint16_t*>(g.out)[o] = bf16_of(silu_mul(gv, uv));
-        else g.out[o] = silu_mul(gv, uv);
-      }
-      return;
-    }
-    for (uint32_t idx = threadIdx.x; idx < kTile * kTile; idx += 256u * KG) {
-      const uint32_t r = idx / kTile, c = idx % kTile, row = m0 + r, col = n0 + c;
-      if (row >= a.m || col >= w.n) continue;
-      float v = reinterpret_cast<const float*>(lds)[idx];
 #pragma unroll
-      for (int g = 1; g < KG; g++) v += reinterpret_cast<const float*>(lds + g * kStageBytes)[idx];
-      if (NORM) v *= inv_rms(r);
-      if (a.partials) {
-        a.partials[((size_t)blockIdx.z * a.m + row) * w.n + col] = v;
-      } else {
-        const size_t o = (size_t)row * w.out_stride + col + w.out_offset;
-        w.out[o] = v + (w.bias ? w.bias[col] : 0.f) + (w.residual ? w.residual[o] : 0.f);
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+          for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bfr[j], acc[i][j], 0, 0, 0);
       }
     }
-    return;
+    __syncthreads();
   }
-
-  // D layout of the 16x16 MFMA: lane l holds rows 4*(l/16) + e, column l % 16.
+  // every group's sums into its own buffers (the last barrier ended the staging), then the groups
+  // added in order by the thread that stores the element
+  float* sums = reinterpret_cast<float*>(lds + group * kStageBytes);
 #pragma unroll
   for (int i = 0; i < 2; i++)
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-      const uint32_t col = n0 + wn + j * 16 + (lane & 15);
-      if (col >= w.n) continue;
-      const float b = (a.partials == nullptr && w.bias) ? w.bias[col] : 0.f;
+    for (int j = 0; j < 2; j++)
 #pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const uint32_t r = wm + i * 16 + 4 * (lane >> 4) + e, row = m0 + r;
-        if (row >= a.m) continue;
-        if (a.partials) {
-          a.partials[((size_t)blockIdx.z * a.m + row) * w.n + col] = acc[i][j][e];
-        } else {
-          const size_t o = (size_t)row * w.out_stride + col + w.out_offset;
-          w.out[o] = (NORM ? acc[i][j][e] * inv_rms(r) : acc[i][j][e]) + b + (w.residual ? w.residual[o] : 0.f);
-        }
-      }
+      for (int e = 0; e < 4; e++)
+        sums[(wm + i * 16 + 4 * (lane >> 4) + e) * kTile + wn + j * 16 + (lane & 15)] = acc[i][j][e];
+  __syncthreads();
+  for (uint32_t idx = threadIdx.x; idx < kTile * kTile; idx += 256u * KG) {
+    const uint32_t r = idx / kTile, c = idx % kTile, row = m0 + r, col = n0 + c;
+    if (row >= a.m || col >= a.n) continue;
+    float v = reinterpret_cast<const float*>(lds)[idx];
+#pragma unroll
+    for (int g = 1; g < KG; g++) v += reinterpret_cast<const float*>(lds + g * kStageBytes)[idx];
+    if (a.partials) {
+      a.partials[((size_t)blockIdx.z * a.m + row) * a.n + col] = v;
+    } else {
+      const size_t o = (size_t)row * a.out_stride + col + a.out_offset;
+      a.out[o] = v + (a.bias ? a.bias[col] : 0.f) + (a.residual ? a.residual[o] : 0.f);
     }
+  }
 }
 
 // The split-K sum: splits added in index order, then the bias.
@@ -570,35 +163,154 @@ __global__ __launch_bounds__(256) void prefill_reduce_kernel(const float* __rest
   }
 }
 
-// Whether a launch maps whole row tiles to each XCD: its grid has no K split and a multiple of 8
-// row tiles, and its column tiles are not a multiple of 8 (with a multiple of 8 the grid's own
-// order already keeps each column tile on one XCD, which suits the wide launches whose weight
-// tiles outweigh their x tiles).
-uint32_t xcd_rows_for(const eg_context* ctx, dim3 grid) {
-  return ctx->prefill_xcd && grid.z == 1 && grid.y % 8 == 0 && grid.x % 8 != 0 ? 1u : 0u;
+// ---- x as bf16 rows -----------------------------------------------------------------------------
+
+// n f32 values (a multiple of 8) rounded to bf16, as the GEMM's own staging rounds them.
+__global__ __launch_bounds__(256) void to_bf16_kernel(const float4* __restrict__ x, uint4* __restrict__ out, size_t n8) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n8; i += (size_t)gridDim.x * blockDim.x) {
+    const float4 a = x[2 * i], b = x[2 * i + 1];
+    out[i] = make_uint4(egd::pack_bf16(a.x, a.y), egd::pack_bf16(a.z, a.w), egd::pack_bf16(b.x, b.y), egd::pack_bf16(b.z, b.w));
+  }
 }
 
-// One launch of the chunked staging with kg groups of 4 waves per workgroup.
-template <bool PAIR, bool NORM, bool ROPE = false, bool XB16 = false>
-void launch_chunked(int encoding, int kg, dim3 grid, hipStream_t stream, const PrefillArgs& a) {
-  const dim3 block(256 * kg);
-#define EG_KG(ENC)                                                                                                  \
-  do {                                                                                                              \
-    if (kg == 4) hipLaunchKernelGGL((prefill_kernel<ENC, true, 4, PAIR, NORM, ROPE, XB16>), grid, block, 0, stream, a);    \
-    else if (kg == 2) hipLaunchKernelGGL((prefill_kernel<ENC, true, 2, PAIR, NORM, ROPE, XB16>), grid, block, 0, stream, a); \
-    else hipLaunchKernelGGL((prefill_kernel<ENC, true, 1, PAIR, NORM, ROPE, XB16>), grid, block, 0, stream, a);            \
-  } while (0)
-  if (encoding == EG_ENC_SIGNED) EG_KG(EG_ENC_SIGNED);
-  else EG_KG(EG_ENC_OFFSET_ZEROS);
-#undef EG_KG
+void to_bf16(eg_context* ctx, const float* x, size_t n, void* out) {
+  const size_t n8 = n / 8;
+  const uint32_t blocks = (uint32_t)std::min<size_t>((n8 + 255) / 256, (size_t)ctx->cu_count * 16);
+  hipLaunchKernelGGL(to_bf16_kernel, dim3(blocks), dim3(256), 0, ctx->stream, reinterpret_cast<const float4*>(x),
+                     static_cast<uint4*>(out), n8);
+}
+
+// The context's buffer for bf16 rows, at least `bytes` long and free for work enqueued next on the
+// current stream: work on another stream that still reads it is waited for (on the device). NULL
+// where there is none: over its bound, during a capture (a graph would keep the address and replay
+// beside other work) or without memory; the caller then takes a tile that stages f32 rows.
+void* bf16_buffer(eg_context* ctx, uint64_t bytes) {
+  if (bytes > eg::kRowsBytes || ctx->capturing) return nullptr;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone) return nullptr;
+  if (ctx->rows_bytes < bytes) {
+    // growing: hipFree waits for the device
+    if (ctx->rows) (void)hipFree(ctx->rows);
+    ctx->rows = nullptr;
+    ctx->rows_bytes = 0;
+    const uint64_t size = std::min<uint64_t>(eg::kRowsBytes, (bytes + (8u << 20) - 1) / (8u << 20) * (8u << 20));
+    if (!ctx->rows_done && hipEventCreateWithFlags(&ctx->rows_done, hipEventDisableTiming) != hipSuccess) {
+      ctx->rows_done = nullptr;
+      return nullptr;
+    }
+    if (hipMalloc(&ctx->rows, size) != hipSuccess) {
+      ctx->rows = nullptr;
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    ctx->rows_bytes = size;
+  }
+  return hipStreamWaitEvent(ctx->stream, ctx->rows_done, 0) == hipSuccess ? ctx->rows : nullptr;
+}
+
+// ---- the choice of a tile -----------------------------------------------------------------------
+
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
+uint64_t tile_count(const Tile& t, uint32_t m, uint64_t cols) {
+  return ((cols + t.wn - 1) / t.wn) * ((m + t.rows() - 1) / t.rows());
+}
+
+// The tile of a launch over m rows, `cols` 64-column tiles and k: the smallest that still covers the
+// matrix in one workgroup per CU (a second round of these workgroups costs more than larger tiles),
+// and the largest where none does. Large tiles spread the dequantization over more rows; small ones
+// fill the device and, with four groups of waves on alternate chunks of K, shorten the serial chain.
+// Measured on MI355X with bf16 rows of x (us; int4 sym at K = 896, ref format else):
+//                        32x64  64x64  64x128  64x256  128x128  128x256
+//     512 x  896 x  896    7.6    8.6    11.4       -        -        -   (224, 112, 56 tiles)
+//    1024 x  896 x  896    9.4    9.0    11.7    15.3        -        -   (448, 224, 112, 64)
+//     128 x 9728 x  896   12.5   15.4    11.9    15.3        -        -   (608, 304, 152, 76)
+//     256 x 9728 x  896   18.7   22.1    16.8    16.1     17.5     23.0   (1216, 608, 304, 152, 152, 76)
+//     512 x 9728 x  896      -      -    25.7    24.6     32.5     24.6   (-, -, 608, 304, 304, 152)
+//    2048 x  896 x 4864   63.2   61.0    41.6    45.5     44.2     41.9   (deep 64x128: 224 tiles)
+//    1024 x 4096 x 4096      -      -    75.3    75.6     54.5     59.4   (-, -, 512, 256, 256, 128)
+//    2048 x 4096 x 11008     -      -       -   305.8    233.1    213.5   (-, -, -, 512, 512, 256)
+// K from 2048 (16 chunks) is long: 64 x 128 then takes eight waves and deeper chunks (41.6 against 54.4 us
+// at 2048 x 896 x 4864; at K = 896 the four-wave form, 12.6 against 13.9 us for f32 rows at 256 x 4864),
+// and 128 x 128 comes before 64 x 256, whose weights are dequantized for half the rows. Blocks of 16
+// codes need the 64-deep chunks.
+Tile tile_for(const eg_context* ctx, uint32_t m, uint64_t cols, uint32_t k, uint32_t bs) {
+  if (ctx->gemm_tile[0]) return Tile{ctx->gemm_tile[0], ctx->gemm_tile[1], ctx->gemm_tile[2], ctx->gemm_tile[3]};
+  const uint64_t cus = (uint64_t)ctx->cu_count;
+  const bool deep = k >= 2048;
+  auto fits = [&](const Tile& t) { return tile_count(t, m, cols) <= cus; };
+  if (bs < 32) return fits(kTile32x64Fine) ? kTile32x64Fine : kTile64x128;
+  // two 32 x 64 workgroups fit on a CU: they may outnumber the CUs a little; over a long K they only
+  // pay where the grid is split anyway
+  if (tile_count(kTile32x64, m, cols) <= (deep ? cus / 2 : cus * 5 / 4)) return kTile32x64;
+  if (fits(kTile64x64)) return kTile64x64;
+  if (fits(kTile64x128)) return deep ? kTile64x128Deep : kTile64x128;
+  if (deep && fits(kTile128x128)) return kTile128x128;
+  if (!deep && fits(kTile64x256)) return kTile64x256;
+  return kTile128x256;
+}
+
+// Ranges K is split into over the grid: where the tiles leave CUs idle over a long K, down to one
+// chunk per group of waves. The partial sums cost a second launch.
+uint64_t splits_for(const eg_context* ctx, const Tile& t, uint32_t m, uint64_t cols, uint32_t k) {
+  if (ctx->gemm_tile[4]) return (uint64_t)ctx->gemm_tile[4];
+  const uint64_t tiles = tile_count(t, m, cols), chunks = (k + t.bk - 1) / t.bk;
+  if (k < 2048 || tiles >= (uint64_t)ctx->cu_count) return 1;
+  return std::max<uint64_t>(1, std::min<uint64_t>(ctx->cu_count / tiles, chunks / t.kg));
+}
+
+// How a launch takes f32 rows of x (*x, m rows of k): the largest tiles take bf16 rows, rounded into
+// `scratch` (nullable; m k halves, 16-byte aligned) or the context's buffer; without either the tile
+// becomes 64 x 256, which stages f32 rows. Measured (MI355X): 2048 x 11008 x 4096 237 us with the rounding
+// launch, 361 with 64 x 256 on f32 rows.
+int stage_f32(eg_context* ctx, const void** x, uint32_t m, uint32_t k, void* scratch, Tile* t, bool* in_rows) {
+  *in_rows = false;
+  if (!t->bf16_only()) return kXF32;
+  void* rows = scratch;
+  if (!rows) {
+    rows = bf16_buffer(ctx, (uint64_t)m * k * 2);
+    *in_rows = rows != nullptr;
+  }
+  if (!rows) {
+    *t = kTile64x256;
+    return kXF32;
+  }
+  to_bf16(ctx, static_cast<const float*>(*x), (size_t)m * k, rows);
+  *x = rows;
+  return kXBf16;
+}
+
+// After the launch that read the context's bf16 rows.
+int rows_used(eg_context* ctx, bool in_rows) {
+  if (!in_rows) return EG_OK;
+  const hipError_t err = hipEventRecord(ctx->rows_done, ctx->stream);
+  return err == hipSuccess ? EG_OK : eg::hip_fail(ctx, err, "matmul_q4_prefill");
+}
+
+// The workgroup grid of a tile over m rows and `cols` 64-column tiles.
+void set_grid(const eg_context* ctx, Args& a, const Tile& t, uint64_t cols) {
+  a.tiles_x = (uint32_t)((cols + t.wn - 1) / t.wn);
+  a.tiles_y = (a.m + t.rows() - 1) / t.rows();
+  a.xcd = ctx->prefill_xcd ? 1u : 0u;
+}
+
+int launch_tile(eg_context* ctx, const char* op, KernelFn fn, const Args& a, const Tile& t, uint32_t splits) {
+  if (!fn) return eg::fail(ctx, EG_ERR_INVALID, "%s: no kernel for tile %d,%d,%d,%d", op, t.bk, t.mf, t.wn, t.kg);
+  hipLaunchKernelGGL(fn, dim3(a.tiles_x * a.tiles_y, splits), dim3(64 * t.wn * t.kg), 0, ctx->stream, a);
+  return EG_OK;
+}
+
+// Whether a matrix's outputs (and residual) take 16-byte accesses.
+bool vector_out(const Mat& w) {
+  return w.n % 4 == 0 && w.out_stride % 4 == 0 && w.out_offset % 4 == 0 && aligned16(w.out) && aligned16(w.residual);
 }
 
 }  // namespace
 
 bool eg::prefill_chunked(uint32_t m, uint32_t n, uint32_t k, uint32_t bs, int bits, const void* x,
                          const uint32_t* packed) {
-  return bits == 4 && k % 32 == 0 && bs % 16 == 0 && (bs & (bs - 1)) == 0 && k % 4 == 0 &&
-         (uint64_t)m * k * 4 < kOutside && (uint64_t)n * k / 2 < kOutside &&
+  return (bits == 4 || bits == 8) && k % 32 == 0 && bs % 16 == 0 && (bs & (bs - 1)) == 0 &&
+         (uint64_t)m * k * 4 < kOutside && (uint64_t)n * k / 8 * bits < kOutside &&
          (reinterpret_cast<uintptr_t>(packed) & 7u) == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
 }
 
@@ -629,60 +341,66 @@ int eg::prefill_gemm(eg_context* ctx, const float* x, const uint32_t* packed, co
   if (m == 0 || n == 0) return EG_OK;
   const uint32_t tiles_n = (n + kTile - 1) / kTile, tiles_m = (m + kTile - 1) / kTile;
   if (tiles_m > 65535) return eg::fail(ctx, EG_ERR_RANGE, "%s: m %u needs %u row tiles, over 65535", op, m, tiles_m);
-  // Groups per workgroup: a grid of at least one tile per CU runs one-group workgroups (three
-  // fit on a CU, so a second round of tiles overlaps the first); a smaller grid runs four groups
-  // per workgroup (one per CU), whose 16 waves work through the tile's K blocks four at a time
-  // (measured at M = 128: gate 11.4 -> 8.3 us; at M = 256 the 304 gate tiles would need a
-  // second round of 1024-thread workgroups: 14.6 -> 16.3 us).
-  const uint64_t tiles = (uint64_t)tiles_n * tiles_m;
-  const uint64_t blocks = (k + kBK - 1) / kBK;
-  const int kg = ctx->prefill_groups ? ctx->prefill_groups : (tiles >= (uint64_t)ctx->cu_count ? 1 : 4);
-  // Split K only where the tile grid leaves most CUs idle over a long reduction (the down
-  // projection: 4 x 14 tiles at M = 256, 76 blocks deep): the partial sums cost a second
-  // launch, so the split must save more block iterations than that launch costs. Four-group
-  // workgroups keep the split grid within one workgroup per CU and at least two blocks per
-  // group. The f32 partials live in the context's workspace.
-  uint64_t splits = 1;
-  if (blocks >= 32 && tiles < (uint64_t)ctx->cu_count)
-    splits = kg == 1 ? std::min<uint64_t>((ctx->cu_count + tiles - 1) / tiles, blocks / 8)
-                     : std::min<uint64_t>(ctx->cu_count / tiles, blocks / (2 * (uint64_t)kg));
-  splits = std::min<uint64_t>(splits, std::max<uint64_t>(1, eg::kPartialsBytes / ((uint64_t)m * n * 4)));
-  splits = std::max<uint64_t>(1, std::min<uint64_t>(splits, 65535));
-  uint32_t k_per_split = (uint32_t)((((uint64_t)k + splits - 1) / splits + kBK - 1) / kBK * kBK);
-  splits = (k + k_per_split - 1) / k_per_split;
-  const bool split = splits > 1;
-  PrefillArgs a{x, split ? reinterpret_cast<float*>(eg::partials(ctx)) : nullptr, m, k, bs, dims->blocks_per_row,
-                k_per_split, bits, (uint32_t)__builtin_ctz(bs), 1u, nullptr, 0.f, nullptr, nullptr, nullptr, nullptr,
-                0u, 0u, 0u, 0u, 0u, {}};
-  a.mats[0] = PrefillMat{packed, scales, encoding == EG_ENC_SIGNED ? nullptr : zeros, dims->use_bias ? bias : nullptr,
-                         residual, out, n, dims->out_stride, dims->out_offset, tiles_n};
-  const dim3 grid(tiles_n, tiles_m, (uint32_t)splits);
-  a.xcd_rows = xcd_rows_for(ctx, grid);
   const bool chunked = eg::prefill_chunked(m, n, k, bs, bits, x, packed);
   if (x_bf16 && !chunked)
     return eg::fail(ctx, EG_ERR_INVALID, "%s: bf16 rows of x need the chunked staging", op);
-  const dim3 block(256 * kg);
-#define EG_PREFILL_LAUNCH(ENC, CH)                                                                        \
-  do {                                                                                                    \
-    if (kg == 4) hipLaunchKernelGGL((prefill_kernel<ENC, CH, 4>), grid, block, 0, ctx->stream, a);        \
-    else if (kg == 2) hipLaunchKernelGGL((prefill_kernel<ENC, CH, 2>), grid, block, 0, ctx->stream, a);   \
-    else hipLaunchKernelGGL((prefill_kernel<ENC, CH, 1>), grid, block, 0, ctx->stream, a);                \
-  } while (0)
-  if (x_bf16) {
-    launch_chunked<false, false, false, true>(encoding, kg, grid, ctx->stream, a);
-  } else if (encoding == EG_ENC_SIGNED) {
-    if (chunked) EG_PREFILL_LAUNCH(EG_ENC_SIGNED, true);
-    else EG_PREFILL_LAUNCH(EG_ENC_SIGNED, false);
+  // Split K only where the tile grid leaves most CUs idle over a long reduction: the partial sums
+  // cost a second launch. They live in the context's workspace.
+  Tile t{};
+  uint64_t splits = 1;
+  uint32_t step = kBK;
+  int kg = 1;
+  if (chunked) {
+    t = tile_for(ctx, m, tiles_n, k, bs);
+    splits = splits_for(ctx, t, m, tiles_n, k);
+    step = t.bk;
   } else {
-    if (chunked) EG_PREFILL_LAUNCH(EG_ENC_OFFSET_ZEROS, true);
-    else EG_PREFILL_LAUNCH(EG_ENC_OFFSET_ZEROS, false);
+    // four groups of waves where the grid holds under a tile per CU, else one
+    const uint64_t tiles = (uint64_t)tiles_n * tiles_m, blocks = (k + kBK - 1) / kBK;
+    kg = tiles >= (uint64_t)ctx->cu_count ? 1 : 4;
+    if (blocks >= 32 && kg == 4) splits = std::min<uint64_t>(ctx->cu_count / tiles, blocks / 8);
   }
-#undef EG_PREFILL_LAUNCH
-  if (split) {
+  splits = std::min<uint64_t>(splits, std::max<uint64_t>(1, eg::kPartialsBytes / ((uint64_t)m * n * 4)));
+  splits = std::max<uint64_t>(1, std::min<uint64_t>(splits, 65535));
+  const uint32_t k_per_split = (uint32_t)((((uint64_t)k + splits - 1) / splits + step - 1) / step * step);
+  splits = (k + k_per_split - 1) / k_per_split;
+  float* const partials = splits > 1 ? reinterpret_cast<float*>(eg::partials(ctx)) : nullptr;
+  const float* const use_bias = dims->use_bias ? bias : nullptr;
+  if (chunked) {
+    Args a{};
+    bool in_rows = false;
+    const void* rows = x;
+    const int xm = x_bf16 ? (int)kXBf16 : stage_f32(ctx, &rows, m, k, nullptr, &t, &in_rows);
+    a.x = rows;
+    a.partials = partials;
+    a.m = m;
+    a.k = k;
+    a.block_shift = (uint32_t)__builtin_ctz(bs);
+    a.blocks_per_row = dims->blocks_per_row;
+    a.k_per_split = k_per_split;
+    a.nmats = 1;
+    a.mats[0] = Mat{packed, scales, encoding == EG_ENC_SIGNED ? nullptr : zeros, use_bias, residual, out, n,
+                    dims->out_stride, dims->out_offset, tiles_n};
+    a.vec = partials ? n % 4 == 0 : vector_out(a.mats[0]);
+    set_grid(ctx, a, t, tiles_n);
+    const KernelFn fn = xm == kXBf16 ? pick_store_bf16(encoding, bits, t) : pick_store_f32(encoding, bits, t);
+    int st = launch_tile(ctx, op, fn, a, t, (uint32_t)splits);
+    if (st == EG_OK) st = rows_used(ctx, in_rows);
+    if (st != EG_OK) return st;
+  } else {
+    const ElementArgs a{x, packed, scales, encoding == EG_ENC_SIGNED ? nullptr : zeros, use_bias, residual, out, partials,
+                        m, n, k, bs, dims->blocks_per_row, k_per_split, dims->out_stride, dims->out_offset, bits};
+    const dim3 grid(tiles_n, tiles_m, (uint32_t)splits), block(256 * kg);
+    const auto fn = encoding == EG_ENC_SIGNED ? (kg == 4 ? element_kernel<EG_ENC_SIGNED, 4> : element_kernel<EG_ENC_SIGNED, 1>)
+                                              : (kg == 4 ? element_kernel<EG_ENC_OFFSET_ZEROS, 4>
+                                                         : element_kernel<EG_ENC_OFFSET_ZEROS, 1>);
+    hipLaunchKernelGGL(fn, grid, block, 0, ctx->stream, a);
+  }
+  if (partials) {
     const uint64_t total = (uint64_t)m * n;
     const uint32_t blocks = (uint32_t)std::min<uint64_t>((total + 255) / 256, (uint64_t)ctx->cu_count * 8);
-    hipLaunchKernelGGL(prefill_reduce_kernel, dim3(blocks), dim3(256), 0, ctx->stream, a.partials, a.mats[0].bias, residual,
-                       out, m, n, (uint32_t)splits, dims->out_stride, dims->out_offset);
+    hipLaunchKernelGGL(prefill_reduce_kernel, dim3(blocks), dim3(256), 0, ctx->stream, partials, use_bias, residual, out,
+                       m, n, (uint32_t)splits, dims->out_stride, dims->out_offset);
   }
   return eg::check_launch(ctx, op);
 }
@@ -690,45 +408,54 @@ int eg::prefill_gemm(eg_context* ctx, const float* x, const uint32_t* packed, co
 namespace {
 
 // Whether matrices sharing x run in ONE launch: the chunked staging takes every one of them and
-// no K split is wanted. Sets the total of their 64-column tiles.
+// no K split is wanted (K under 2048). Sets the total of their 64-column tiles, and the number the
+// launch's tile is chosen for: matrices of one shape take the tile that one of them alone takes, so
+// that gate and up as a pair, in one launch and on their own give the same bits (4% slower at 256
+// rows of the pair than its own best tile, equal from 512); others their total.
 bool one_launch(const float* x, uint32_t m, uint32_t k, uint32_t block_size, int encoding, int bits,
-                const eg::PrefillMatrix* mats, uint32_t count, uint64_t* tiles_n) {
+                const eg::PrefillMatrix* mats, uint32_t count, uint64_t* tiles_n, uint64_t* tile_cols) {
   bool ok = count >= 1 && count <= kMaxSegs && m > 0 && x && bits == 4 &&
             (encoding == EG_ENC_SIGNED || encoding == EG_ENC_OFFSET_ZEROS) && block_size >= 16 &&
             (block_size & (block_size - 1)) == 0 && k % block_size == 0 && k % 32 == 0 &&
             (k + kBK - 1) / kBK < 32 && (uint64_t)m * k * 4 < kOutside && (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
   *tiles_n = 0;
+  bool same = true;
   for (uint32_t i = 0; ok && i < count; i++) {
     const eg::PrefillMatrix& w = mats[i];
     ok = w.n > 0 && w.packed && w.scales && w.out && (encoding == EG_ENC_SIGNED || w.zeros) &&
          (m == 1 || w.out_stride >= w.n) && (uint64_t)w.n * k / 2 < kOutside &&
          (uint64_t)w.n * (k / block_size) < (1ull << 32) && (reinterpret_cast<uintptr_t>(w.packed) & 7u) == 0;
     *tiles_n += (w.n + kTile - 1) / kTile;
+    if (w.n != mats[0].n) same = false;
   }
+  *tile_cols = same && count ? *tiles_n / count : *tiles_n;
   return ok && *tiles_n <= 0x7FFFFFFFull && (m + kTile - 1) / kTile <= 65535;
 }
 
-// Groups per workgroup for a tile grid: one where the grid holds at least a tile per CU, else four.
-int groups_for(const eg_context* ctx, uint64_t tiles) {
-  return ctx->prefill_groups ? ctx->prefill_groups : (tiles >= (uint64_t)ctx->cu_count ? 1 : 4);
+// Whether a launch folds the rows' RMSNorm in: only under one 64 x 64 tile per CU (latency-bound),
+// where the extra staging work (the weight multiply and the squares) is hidden; a launch that fills
+// the device is bound by that work, and a separate rmsnorm_rows launch costs less. (These launches
+// take tiles of up to 64 x 128.)
+bool fold_norm(const eg_context* ctx, uint32_t m, uint64_t cols, const float* norm) {
+  return norm && aligned16(norm) && cols * ((m + kTile - 1) / kTile) < (uint64_t)ctx->cu_count;
 }
 
-// Whether a launch folds the rows' RMSNorm in: only with four-group workgroups (a grid under one
-// tile per CU, latency-bound), where the extra staging work (the weight multiply and the squares,
-// 32 VALU operations per thread and block) is hidden; a launch that fills the device is bound by
-// that work, and a separate rmsnorm_rows launch costs less there (measured at 2048 rows: the
-// gate|up pair 94 -> 128 us with the norm folded in, against 5.5 us for rmsnorm_rows).
-bool fold_norm(const eg_context* ctx, uint64_t tiles, const float* norm) {
-  return norm && (reinterpret_cast<uintptr_t>(norm) & 15u) == 0 && groups_for(ctx, tiles) == 4;
-}
-
-// The matrices (one_launch accepted them) as one chunked launch; norm non-NULL folds the rows'
-// RMSNorm into it.
-int launch_multi(eg_context* ctx, const float* x, uint32_t m, uint32_t k, uint32_t block_size, int encoding, int bits,
-                 const eg::PrefillMatrix* mats, uint32_t count, uint64_t tiles_n, const float* norm, float eps,
-                 const eg::PrefillRope* rope = nullptr, bool x_bf16 = false) {
-  PrefillArgs a{x, nullptr, m, k, block_size, k / block_size, k, bits, (uint32_t)__builtin_ctz(block_size), count,
-                norm, eps, nullptr, nullptr, nullptr, nullptr, 0u, 0u, 0u, 0u, 0u, {}};
+// The matrices (one_launch accepted them) as one launch; xm says how x is staged (kXNorm with
+// norm and eps: the rows' RMSNorm folded in).
+int launch_multi(eg_context* ctx, const void* x, uint32_t m, uint32_t k, uint32_t block_size, int encoding,
+                 const eg::PrefillMatrix* mats, uint32_t count, uint64_t cols, int xm, int epi, const Tile& t,
+                 const float* norm, float eps, const eg::PrefillRope* rope = nullptr, bool out_bf16 = false) {
+  Args a{};
+  a.x = x;
+  a.m = m;
+  a.k = k;
+  a.block_shift = (uint32_t)__builtin_ctz(block_size);
+  a.blocks_per_row = k / block_size;
+  a.k_per_split = k;
+  a.nmats = count;
+  a.norm = norm;
+  a.eps = eps;
+  a.out_bf16 = out_bf16 ? 1u : 0u;
   if (rope) {
     a.rope = rope->table;
     a.q_rope = rope->q_rope;
@@ -739,28 +466,46 @@ int launch_multi(eg_context* ctx, const float* x, uint32_t m, uint32_t k, uint32
     a.kv_heads = rope->kv_heads;
   }
   uint32_t end = 0;
+  a.vec = 1;
   for (uint32_t i = 0; i < count; i++) {
     const eg::PrefillMatrix& w = mats[i];
-    end += (w.n + kTile - 1) / kTile;
-    a.mats[i] = PrefillMat{w.packed, w.scales, encoding == EG_ENC_SIGNED ? nullptr : w.zeros, w.bias, w.residual,
-                           w.out, w.n, w.out_stride, w.out_offset, end};
+    end = epi == kPair ? (uint32_t)cols : end + (w.n + kTile - 1) / kTile;
+    a.mats[i] = Mat{w.packed, w.scales, encoding == EG_ENC_SIGNED ? nullptr : w.zeros, w.bias, w.residual,
+                    w.out, w.n, w.out_stride, w.out_offset, end};
+    if (!vector_out(a.mats[i])) a.vec = 0;
   }
-  const uint64_t tiles_m = (m + kTile - 1) / kTile;
-  const int kg = groups_for(ctx, tiles_n * tiles_m);
-  const dim3 grid((uint32_t)tiles_n, (uint32_t)tiles_m, 1);
-  a.xcd_rows = xcd_rows_for(ctx, grid);
-  if (rope) {
-    if (norm) launch_chunked<false, true, true>(encoding, kg, grid, ctx->stream, a);
-    else if (x_bf16) launch_chunked<false, false, true, true>(encoding, kg, grid, ctx->stream, a);
-    else launch_chunked<false, false, true>(encoding, kg, grid, ctx->stream, a);
-  } else if (norm) {
-    launch_chunked<false, true>(encoding, kg, grid, ctx->stream, a);
-  } else if (x_bf16) {
-    launch_chunked<false, false, false, true>(encoding, kg, grid, ctx->stream, a);
-  } else {
-    launch_chunked<false, false>(encoding, kg, grid, ctx->stream, a);
+  set_grid(ctx, a, t, cols);
+  KernelFn fn = nullptr;
+  if (epi == kRope) fn = pick_rope(encoding, xm, t);
+  else if (epi == kPair) fn = pick_pair(encoding, xm, t);
+  else if (xm == kXNorm) fn = pick_store_norm(encoding, 4, t);
+  else fn = xm == kXBf16 ? pick_store_bf16(encoding, 4, t) : pick_store_f32(encoding, 4, t);
+  const int st = launch_tile(ctx, "matmul_q4_prefill", fn, a, t, 1);
+  return st != EG_OK ? st : eg::check_launch(ctx, "matmul_q4_prefill");
+}
+
+// x of a launch of tile *t: the rows' RMSNorm folded into it where that pays (kXNorm), else rmsnorm_rows
+// into `normed` - as bf16 rows where the context stages them - and f32 rows as stage_f32 takes them.
+// Sets *x, *xm and *in_rows.
+int prepare_x(eg_context* ctx, const void** x, uint32_t m, uint32_t k, uint64_t cols, Tile* t, const float* norm,
+              float eps, float* normed, void* scratch, int* xm, bool* in_rows) {
+  *in_rows = false;
+  if (fold_norm(ctx, m, cols, norm)) {
+    *xm = kXNorm;
+    return EG_OK;
   }
-  return eg::check_launch(ctx, "matmul_q4_prefill");
+  if (norm) {
+    if (!normed) return eg::fail(ctx, EG_ERR_INVALID, "matmul_q4_prefill: RMSNorm needs a buffer for the normed rows");
+    const int st = eg::rmsnorm_rows(ctx, static_cast<const float*>(*x), norm, m, k, eps, normed, ctx->prefill_xb16);
+    if (st != EG_OK) return st;
+    *x = normed;
+    if (ctx->prefill_xb16) {
+      *xm = kXBf16;
+      return EG_OK;
+    }
+  }
+  *xm = stage_f32(ctx, x, m, k, scratch, t, in_rows);
+  return EG_OK;
 }
 
 }  // namespace
@@ -771,23 +516,26 @@ int eg::prefill_gemm_multi(eg_context* ctx, const float* x, uint32_t m, uint32_t
   const char* op = "matmul_q4_prefill";
   if (!ctx) return eg::fail(nullptr, EG_ERR_INVALID, "%s: ctx is NULL", op);
   if (count > 0 && !mats) return eg::fail(ctx, EG_ERR_INVALID, "%s: NULL matrix list", op);
-  uint64_t tiles_n = 0;
-  const uint64_t tiles_m = (m + kTile - 1) / kTile;
+  uint64_t cols = 0, tile_cols = 0;
+  // One launch where the chunked staging takes every matrix and no matrix would split K;
+  // otherwise (and for anything the single path must reject with its own message) one each.
+  if ((count >= 2 || norm) && one_launch(x, m, k, block_size, encoding, bits, mats, count, &cols, &tile_cols)) {
+    Tile t = tile_for(ctx, m, tile_cols, k, block_size);
+    int xm = kXF32;
+    bool in_rows = false;
+    const void* rows = x;
+    int st = prepare_x(ctx, &rows, m, k, cols, &t, norm, eps, normed, nullptr, &xm, &in_rows);
+    if (st == EG_OK) st = launch_multi(ctx, rows, m, k, block_size, encoding, mats, count, cols, xm, kStore, t, norm, eps);
+    return st == EG_OK ? rows_used(ctx, in_rows) : st;
+  }
   if (norm) {
-    // RMSNorm folded into the one launch where that pays (fold_norm); otherwise rmsnorm_rows
-    // into `normed` (as bf16 rows when the one launch stages them) and the launches below on it
-    const bool one = one_launch(x, m, k, block_size, encoding, bits, mats, count, &tiles_n);
-    if (one && fold_norm(ctx, tiles_n * tiles_m, norm))
-      return launch_multi(ctx, x, m, k, block_size, encoding, bits, mats, count, tiles_n, norm, eps);
     if (!normed) return eg::fail(ctx, EG_ERR_INVALID, "%s: RMSNorm needs a buffer for the normed rows", op);
-    const bool xb = one && ctx->prefill_xb16;
-    const int st = eg::rmsnorm_rows(ctx, x, norm, m, k, eps, normed, xb);
+    const int st = eg::rmsnorm_rows(ctx, x, norm, m, k, eps, normed, false);
     if (st != EG_OK) return st;
-    if (xb) return launch_multi(ctx, normed, m, k, block_size, encoding, bits, mats, count, tiles_n, nullptr, 0.f,
-                                nullptr, true);
     x = normed;
   }
-  auto one = [&](const PrefillMatrix& w) {
+  for (uint32_t i = 0; i < count; i++) {
+    const PrefillMatrix& w = mats[i];
     eg_matmul_q4_dims dm{};
     dm.m = m;
     dm.n = w.n;
@@ -797,19 +545,10 @@ int eg::prefill_gemm_multi(eg_context* ctx, const float* x, uint32_t m, uint32_t
     dm.blocks_per_row = block_size ? k / block_size : 0;
     dm.out_stride = w.out_stride;
     dm.out_offset = w.out_offset;
-    return eg::prefill_gemm(ctx, x, w.packed, w.scales, w.zeros, w.bias, w.residual, w.out, &dm, encoding, bits);
-  };
-  // One launch where the chunked staging takes every matrix and no matrix would split K;
-  // otherwise (and for anything the single path must reject with its own message) one each.
-  if (count < 2 || !one_launch(x, m, k, block_size, encoding, bits, mats, count, &tiles_n)) {
-    for (uint32_t i = 0; i < count; i++) {
-      const int st = one(mats[i]);
-      if (st != EG_OK) return st;
-    }
-    return EG_OK;
+    const int st = eg::prefill_gemm(ctx, x, w.packed, w.scales, w.zeros, w.bias, w.residual, w.out, &dm, encoding, bits);
+    if (st != EG_OK) return st;
   }
-  (void)tiles_m;
-  return launch_multi(ctx, x, m, k, block_size, encoding, bits, mats, count, tiles_n, nullptr, 0.f);
+  return EG_OK;
 }
 
 int eg::prefill_qkv_rope(eg_context* ctx, const float* x, uint32_t m, uint32_t k, uint32_t block_size, int encoding,
@@ -817,23 +556,21 @@ int eg::prefill_qkv_rope(eg_context* ctx, const float* x, uint32_t m, uint32_t k
                          const PrefillRope& rope, bool* done) {
   *done = false;
   if (!ctx || !mats || !ctx->prefill_rope || m == 0) return EG_OK;
-  uint64_t tiles_n = 0;
-  if (!rope.table || !rope.q_rope || !rope.k_cache || !rope.v_cache || mats[0].n != rope.q_heads * kTile ||
+  uint64_t cols = 0, tile_cols = 0;
+  if (!rope.table || !rope.q_rope || !rope.k_cache || !rope.v_cache || !aligned16(rope.q_rope) ||
+      !aligned16(rope.k_cache) || !aligned16(rope.v_cache) || mats[0].n != rope.q_heads * kTile ||
       mats[1].n != rope.kv_heads * kTile || mats[2].n != rope.kv_heads * kTile ||
-      !one_launch(x, m, k, block_size, encoding, bits, mats, 3, &tiles_n))
+      !one_launch(x, m, k, block_size, encoding, bits, mats, 3, &cols, &tile_cols))
     return EG_OK;
-  const uint64_t tiles_m = (m + kTile - 1) / kTile;
-  bool xb = false;
-  if (norm && !fold_norm(ctx, tiles_n * tiles_m, norm)) {
-    if (!normed) return eg::fail(ctx, EG_ERR_INVALID, "matmul_q4_prefill: RMSNorm needs a buffer for the normed rows");
-    xb = ctx->prefill_xb16;
-    const int st = eg::rmsnorm_rows(ctx, x, norm, m, k, eps, normed, xb);
-    if (st != EG_OK) return st;
-    x = normed;
-    norm = nullptr;
-  }
+  Tile t = tile_for(ctx, m, tile_cols, k, block_size);
+  int xm = kXF32;
+  bool in_rows = false;
+  const void* rows = x;
+  int st = prepare_x(ctx, &rows, m, k, cols, &t, norm, eps, normed, nullptr, &xm, &in_rows);
+  if (st != EG_OK) return st;
   *done = true;
-  return launch_multi(ctx, x, m, k, block_size, encoding, bits, mats, 3, tiles_n, norm, eps, &rope, xb);
+  st = launch_multi(ctx, rows, m, k, block_size, encoding, mats, 3, cols, xm, kRope, t, norm, eps, &rope);
+  return st == EG_OK ? rows_used(ctx, in_rows) : st;
 }
 
 int eg::prefill_gemm_swiglu(eg_context* ctx, const float* x, uint32_t m, uint32_t k, uint32_t block_size,
@@ -844,11 +581,12 @@ int eg::prefill_gemm_swiglu(eg_context* ctx, const float* x, uint32_t m, uint32_
   if (!out || !scratch || gate.n != up.n)
     return eg::fail(ctx, EG_ERR_INVALID, "%s: SwiGLU pair needs matching gate and up and two outputs", op);
   const uint32_t n = gate.n;
-  // the pair as ONE launch of paired tiles where the chunked staging takes both and K is short
+  // the pair as ONE launch of paired tiles where the chunked staging takes both, K is short and there are no biases
   const PrefillMatrix pair[2] = {{gate.packed, gate.scales, gate.zeros, gate.bias, nullptr, out, n, n, 0},
                                  {up.packed, up.scales, up.zeros, up.bias, nullptr, out, n, n, 0}};
-  uint64_t tiles_n = 0;
-  if (n == 0 || m == 0 || !ctx->prefill_pair || !one_launch(x, m, k, block_size, encoding, bits, pair, 2, &tiles_n)) {
+  uint64_t cols = 0, tile_cols = 0;
+  if (n == 0 || m == 0 || !ctx->prefill_pair || gate.bias || up.bias ||
+      !one_launch(x, m, k, block_size, encoding, bits, pair, 2, &cols, &tile_cols)) {
     // otherwise gate | up side by side in the scratch rows, then SiLU(gate) * up
     const PrefillMatrix gu[2] = {{gate.packed, gate.scales, gate.zeros, gate.bias, nullptr, scratch, n, 2 * n, 0},
                                  {up.packed, up.scales, up.zeros, up.bias, nullptr, scratch, n, 2 * n, n}};
@@ -856,31 +594,17 @@ int eg::prefill_gemm_swiglu(eg_context* ctx, const float* x, uint32_t m, uint32_
     if (st == EG_OK && m > 0 && n > 0) st = eg::silu_mul_rows(ctx, scratch, m, n, out, out_bf16);
     return st;
   }
-  const uint32_t tiles_x = (n + 31) / 32;
-  const uint64_t tiles_m = (m + kTile - 1) / kTile;
-  const int kg = groups_for(ctx, (uint64_t)tiles_x * tiles_m);
-  bool xb = false;
-  if (norm && !fold_norm(ctx, (uint64_t)tiles_x * tiles_m, norm)) {
-    if (!normed) return eg::fail(ctx, EG_ERR_INVALID, "%s: RMSNorm needs a buffer for the normed rows", op);
-    xb = ctx->prefill_xb16;
-    const int st = eg::rmsnorm_rows(ctx, x, norm, m, k, eps, normed, xb);
-    if (st != EG_OK) return st;
-    x = normed;
-    norm = nullptr;
-  }
-  PrefillArgs a{x, nullptr, m, k, block_size, k / block_size, k, bits, (uint32_t)__builtin_ctz(block_size), 2u,
-                norm, eps, nullptr, nullptr, nullptr, nullptr, 0u, 0u, 0u, out_bf16 ? 1u : 0u, 0u, {}};
-  for (int i = 0; i < 2; i++) {
-    const PrefillMatrix& w = pair[i];
-    a.mats[i] = PrefillMat{w.packed, w.scales, encoding == EG_ENC_SIGNED ? nullptr : w.zeros, w.bias, nullptr,
-                           w.out, n, n, 0, tiles_x};
-  }
-  const dim3 grid(tiles_x, (uint32_t)tiles_m, 1);
-  a.xcd_rows = xcd_rows_for(ctx, grid);
-  if (norm) launch_chunked<true, true>(encoding, kg, grid, ctx->stream, a);
-  else if (xb) launch_chunked<true, false, false, true>(encoding, kg, grid, ctx->stream, a);
-  else launch_chunked<true, false>(encoding, kg, grid, ctx->stream, a);
-  return eg::check_launch(ctx, op);
+  Tile t = tile_for(ctx, m, tile_cols, k, block_size);
+  int xm = kXF32;
+  bool in_rows = false;
+  const void* rows = x;
+  // the scratch rows ([m][2 n] floats) are free here: they hold the bf16 rows of x where those fit
+  void* const spare = (uint64_t)2 * n * 4 >= (uint64_t)k * 2 && aligned16(scratch) ? scratch : nullptr;
+  int st = prepare_x(ctx, &rows, m, k, (n + 31) / 32, &t, norm, eps, normed, spare, &xm, &in_rows);
+  if (st != EG_OK) return st;
+  st = launch_multi(ctx, rows, m, k, block_size, encoding, pair, 2, (n + 31) / 32, xm, kPair, t, norm, eps, nullptr,
+                    out_bf16);
+  return st == EG_OK ? rows_used(ctx, in_rows) : st;
 }
 
 extern "C" int eg_matmul_q4_prefill_swiglu(eg_context* ctx, const float* x, const uint32_t* gate_packed,

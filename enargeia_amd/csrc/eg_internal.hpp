@@ -42,9 +42,14 @@ struct eg_context {
   uint64_t* stamps = nullptr;
   uint32_t stamp_capacity = 0;
   uint32_t stamp_next = 0;
-  // Groups of 4 waves per prefill GEMM workgroup, each on its own K blocks: 0 = chosen per
-  // launch from the tile grid; EG_PREFILL_GROUPS=1, 2 or 4 forces one (for tuning sweeps).
-  int prefill_groups = 0;
+  // The prefill GEMM's tile (BK, MF, WN, KG of its kernel, and the K splits) forced by
+  // EG_PREFILL_TILE="bk,mf,wn,kg[,splits]" for tuning sweeps; zeros: chosen per launch.
+  int gemm_tile[5] = {0, 0, 0, 0, 0};
+  // bf16 rows of a prefill GEMM's f32 x (eg_gemm.hip): grown on use up to eg::kRowsBytes, freed with
+  // the context; the event after its last use.
+  void* rows = nullptr;
+  size_t rows_bytes = 0;
+  hipEvent_t rows_done = nullptr;
   // chunk attention's key split: at most this many 64-key tiles per workgroup, and a small grid
   // split up to this many workgroups per CU
   // the SwiGLU pair as one launch of paired gate|up tiles (false: gate | up, then silu_mul_rows)
@@ -91,6 +96,7 @@ constexpr size_t kWorkspaceBytes = 64u << 20;  // 64 MiB
 inline uint8_t* state(eg_context* ctx) { return ctx->workspace + kStateOffset; }
 inline uint8_t* partials(eg_context* ctx) { return ctx->workspace + kPartialsOffset; }
 constexpr size_t kPartialsBytes = kWorkspaceBytes - kPartialsOffset;
+constexpr size_t kRowsBytes = 64u << 20;  // bound of eg_context::rows
 
 // Second stage of every multi-workgroup argmax: one workgroup reduces `groups` partials
 // (value bits, index) in a fixed order into result = [index, value bits]. A separate launch
@@ -401,6 +407,13 @@ __device__ __forceinline__ float load_f32(__amdgpu_buffer_rsrc_t r, uint32_t off
 }
 __device__ __forceinline__ void store_f32(__amdgpu_buffer_rsrc_t r, uint32_t offset, float v, uint32_t soffset = 0) {
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, offset, soffset, 0);
+}
+
+// 16 bytes per lane from memory straight into LDS: lane l's land at lds + 16 l (`lds` wave-uniform);
+// a lane whose offset is past the end leaves zeros. Counted on vmcnt like any load, and not waited
+// for by a barrier: the wave waits (s_waitcnt vmcnt) before the barrier that publishes the data.
+__device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t r, void* lds, uint32_t offset) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, offset, 0, 0, 0);
 }
 
 // The same accesses with an explicit cache policy: AUX = 0 is the default policy; AUX = kCoherent
