@@ -240,11 +240,12 @@ Tile tile_for(const eg_context* ctx, uint32_t m, uint64_t cols, uint32_t k, uint
   const bool deep = k >= 2048;
   auto fits = [&](const Tile& t) { return tile_count(t, m, cols) <= cus; };
   if (bs < 32) return fits(kTile32x64Fine) ? kTile32x64Fine : kTile64x128;
-  // two 32 x 64 workgroups fit on a CU: they may outnumber the CUs a little; over a long K they only
-  // pay where the grid is split anyway
+  // two workgroups of 32 x 64 (or of 64 x 128) fit on a CU: they may outnumber the CUs a little; over a
+  // long K 32 x 64 only pays where the grid is split anyway
   if (tile_count(kTile32x64, m, cols) <= (deep ? cus / 2 : cus * 5 / 4)) return kTile32x64;
   if (fits(kTile64x64)) return kTile64x64;
-  if (fits(kTile64x128)) return deep ? kTile64x128Deep : kTile64x128;
+  if (deep ? fits(kTile64x128Deep) : tile_count(kTile64x128, m, cols) <= cus * 5 / 4)
+    return deep ? kTile64x128Deep : kTile64x128;
   if (deep && fits(kTile128x128)) return kTile128x128;
   if (!deep && fits(kTile64x256)) return kTile64x256;
   return kTile128x256;
@@ -287,11 +288,17 @@ int rows_used(eg_context* ctx, bool in_rows) {
   return err == hipSuccess ? EG_OK : eg::hip_fail(ctx, err, "matmul_q4_prefill");
 }
 
-// The workgroup grid of a tile over m rows and `cols` 64-column tiles.
-void set_grid(const eg_context* ctx, Args& a, const Tile& t, uint64_t cols) {
+// The workgroup grid of a tile over m rows and `cols` 64-column tiles, and the order its tiles are
+// dealt to the XCDs in: the one whose runs read fewer bytes into an L2 - column-major 1/8 of W and up to
+// all of x, row-major 1/8 of x and up to all of W. (2048 x 896 x 4864, x 20 MB and W 2.4 MB: 44.7 us with
+// column-major runs, 39.9 with row-major ones.)
+void set_grid(const eg_context* ctx, Args& a, const Tile& t, uint64_t cols, int xm, int bits) {
   a.tiles_x = (uint32_t)((cols + t.wn - 1) / t.wn);
   a.tiles_y = (a.m + t.rows() - 1) / t.rows();
-  a.xcd = ctx->prefill_xcd ? 1u : 0u;
+  const double run = (double)a.tiles_x * a.tiles_y / 8.0;
+  const double x = (double)a.m * a.k * (xm == kXBf16 ? 2 : 4), w = (double)cols * kCols * a.k * bits / 8;
+  const double column_major = x * std::min(1.0, run / a.tiles_y) + w / 8, row_major = x / 8 + w * std::min(1.0, run / a.tiles_x);
+  a.xcd = !ctx->prefill_xcd ? 0u : column_major <= row_major ? 1u : 2u;
 }
 
 int launch_tile(eg_context* ctx, const char* op, KernelFn fn, const Args& a, const Tile& t, uint32_t splits) {
@@ -382,7 +389,7 @@ int eg::prefill_gemm(eg_context* ctx, const float* x, const uint32_t* packed, co
     a.mats[0] = Mat{packed, scales, encoding == EG_ENC_SIGNED ? nullptr : zeros, use_bias, residual, out, n,
                     dims->out_stride, dims->out_offset, tiles_n};
     a.vec = partials ? n % 4 == 0 : vector_out(a.mats[0]);
-    set_grid(ctx, a, t, tiles_n);
+    set_grid(ctx, a, t, tiles_n, xm, bits);
     const KernelFn fn = xm == kXBf16 ? pick_store_bf16(encoding, bits, t) : pick_store_f32(encoding, bits, t);
     int st = launch_tile(ctx, op, fn, a, t, (uint32_t)splits);
     if (st == EG_OK) st = rows_used(ctx, in_rows);
@@ -474,7 +481,7 @@ int launch_multi(eg_context* ctx, const void* x, uint32_t m, uint32_t k, uint32_
                     w.out, w.n, w.out_stride, w.out_offset, end};
     if (!vector_out(a.mats[i])) a.vec = 0;
   }
-  set_grid(ctx, a, t, cols);
+  set_grid(ctx, a, t, cols, xm, 4);
   KernelFn fn = nullptr;
   if (epi == kRope) fn = pick_rope(encoding, xm, t);
   else if (epi == kPair) fn = pick_pair(encoding, xm, t);

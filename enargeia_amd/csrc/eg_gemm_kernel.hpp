@@ -57,7 +57,7 @@ struct Args {
   uint32_t m, k, block_shift, blocks_per_row, k_per_split;
   uint32_t tiles_x, tiles_y;  // workgroup tiles
   uint32_t nmats;             // matrices in mats (> 1: no K split)
-  uint32_t xcd;               // tiles dealt to the XCDs in contiguous runs (see tile_of)
+  uint32_t xcd;               // order in which tiles are dealt to the XCDs (see tile_of)
   uint32_t vec;               // outputs (and residuals) take 16-byte accesses, n a multiple of 4
   const float* norm;          // kXNorm: x is RMS-normalised per row with these weights (no K split)
   float eps;
@@ -81,19 +81,21 @@ enum Epilogue { kStore = 0, kPair = 1, kRope = 2 };
 __device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.0f + expf(-g)) * u; }
 
 // Workgroup L's tile. Workgroups go to the 8 XCDs in turn (L on XCD L % 8), each with its own L2.
-// With `xcd` each XCD takes a contiguous run of the tiles in column-major order (all row tiles of a
-// column tile, then the next), so the weights of a column tile are read into one L2 and the rows of
-// x are shared by the run's column tiles; otherwise the grid's own row-major order.
+// With `xcd` each XCD takes a contiguous run of the tiles: in column-major order (1: it reads an
+// eighth of the weights and up to all of x) or row-major (2: an eighth of x and up to all of the
+// weights); otherwise the grid's own row-major order.
 __device__ __forceinline__ void tile_of(const Args& a, uint32_t& tx, uint32_t& ty) {
-  const uint32_t L = blockIdx.x;
+  uint32_t id = blockIdx.x;
   if (a.xcd) {
-    const uint32_t total = a.tiles_x * a.tiles_y, q = total / 8u, r = total % 8u;
-    const uint32_t xcd = L % 8u, id = xcd * q + min(xcd, r) + L / 8u;
+    const uint32_t total = a.tiles_x * a.tiles_y, q = total / 8u, r = total % 8u, xcd = id % 8u;
+    id = xcd * q + min(xcd, r) + id / 8u;
+  }
+  if (a.xcd == 1u) {
     tx = id / a.tiles_y;
     ty = id % a.tiles_y;
   } else {
-    tx = L % a.tiles_x;
-    ty = L / a.tiles_x;
+    tx = id % a.tiles_x;
+    ty = id / a.tiles_x;
   }
 }
 
@@ -416,7 +418,17 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_kernel(Args a) {
   }
 
   // ---- epilogue: unit (i, p) = row fragment i with columns 8 p + 4 g .. +4 of both column fragments --
-  auto finish = [&](uint32_t i, uint32_t p, f32x4 lo, f32x4 hi) {
+  // kRope: cos and sin of unit (i, p)'s four pairs, which the callers read ahead of the sums
+  struct Angles {
+    double2 cs[EPI == kRope ? 4 : 1];
+  };
+  auto angles_of = [&](uint32_t i, uint32_t p, Angles& c) {
+    if (EPI != kRope || si == 2) return;
+    const uint32_t row = min(m0 + 32u * i + lr, a.m - 1);
+#pragma unroll
+    for (int e = 0; e < 4; e++) c.cs[EPI == kRope ? e : 0] = a.rope[(size_t)(a.rope_pos0 + row) * 32u + 8u * p + 4u * g + e];
+  };
+  auto finish = [&](uint32_t i, uint32_t p, f32x4 lo, f32x4 hi, const Angles& an) {
     const uint32_t r = 32u * i + lr, row = m0 + r;
     if (!active || row >= a.m) return;
     if (XM == kXNorm) {
@@ -459,7 +471,7 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_kernel(Args a) {
         x[e] = lo[e] + (w0.bias ? w0.bias[n0 + c + e] : 0.f) + 0.f;
         y[e] = hi[e] + (w0.bias ? w0.bias[n0 + c + 32u + e] : 0.f) + 0.f;
         if (si < 2) {
-          const float2 rr = egd::rotate(x[e], y[e], a.rope[(size_t)(a.rope_pos0 + row) * 32u + c + e]);
+          const float2 rr = egd::rotate(x[e], y[e], an.cs[EPI == kRope ? e : 0]);
           x[e] = rr.x;
           y[e] = rr.y;
         }
@@ -516,7 +528,9 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_kernel(Args a) {
     for (int i = 0; i < MF; i++)
 #pragma unroll
       for (int p = 0; p < 4; p++) {
-        finish(i, p, run(acc[0][i], p), run(acc[1][i], p));
+        Angles an;
+        angles_of(i, p, an);
+        finish(i, p, run(acc[0][i], p), run(acc[1][i], p), an);
         __builtin_amdgcn_sched_barrier(0);  // one unit at a time: together they spill
       }
   } else {
@@ -528,18 +542,21 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_kernel(Args a) {
     for (int f = 0; f < 2; f++)
 #pragma unroll
       for (int u = 0; u < 4 * MF; u++) sums[at(group, f, u)] = run(acc[f][u / 4], u % 4);
+    static_assert(4 * MF % KG == 0, "the groups share the units");
+    Angles an[4 * MF / KG];
+#pragma unroll
+    for (uint32_t v = 0; v < 4u * MF / KG; v++) angles_of((group + v * KG) / 4, (group + v * KG) % 4, an[v]);
     __syncthreads();
 #pragma unroll
-    for (uint32_t v = 0; v < (4u * MF + KG - 1) / KG; v++) {
+    for (uint32_t v = 0; v < 4u * MF / KG; v++) {
       const uint32_t u = group + v * KG;
-      if (4 * MF % KG != 0 && u >= 4u * MF) break;
       f32x4 lo = sums[at(0, 0, u)], hi = sums[at(0, 1, u)];
 #pragma unroll
       for (int q = 1; q < KG; q++) {
         lo += sums[at(q, 0, u)];
         hi += sums[at(q, 1, u)];
       }
-      finish(u / 4, u % 4, lo, hi);
+      finish(u / 4, u % 4, lo, hi, an[v]);
     }
   }
 }
