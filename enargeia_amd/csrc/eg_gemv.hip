@@ -80,6 +80,187 @@ __global__ __launch_bounds__(256) void gemv_generic_kernel(
   }
 }
 
+// One 16-byte chunk's sum of (code - zero) * x, without the sum of x that Codes::dot takes apart (an
+// infinite x then gives what a product per code gives). A code masked into the low ten bits of an
+// f16 1024.0 reads 1024 + code (a high nibble, left in place, 1024 + 16 code); adding -(1024 + zero)
+// leaves code - zero exactly, and v_fma_mix_f32 multiplies that half by the f32 x - by x / 16, staged
+// so, for high nibbles. z: the zero-point.
+template <int BITS, int ENC>
+__device__ __forceinline__ float exact_dot(const egd::u32x4& q, const float (&x)[128 / BITS], uint32_t z) {
+  auto halves = [](uint32_t v) { return __builtin_bit_cast(half2v, v); };
+  const half2v zl = halves((0xE400u | z) * 0x10001u);
+  float a0 = 0.f, a1 = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const uint32_t d = q[i], d8 = d >> 8;
+    if constexpr (BITS == 4) {
+      constexpr uint32_t lo = ENC == EG_ENC_SIGNED ? 0x64086408u : 0x64006400u;
+      constexpr uint32_t hi = ENC == EG_ENC_SIGNED ? 0x64806480u : 0x64006400u;
+      const half2v zh = halves((0xE400u | (z << 4)) * 0x10001u);
+      const half2v c0 = halves((d & 0x000F000Fu) ^ lo) + zl, c1 = halves((d & 0x00F000F0u) ^ hi) + zh;
+      const half2v c2 = halves((d8 & 0x000F000Fu) ^ lo) + zl, c3 = halves((d8 & 0x00F000F0u) ^ hi) + zh;
+      const float* xv = x + 8 * i;
+      a0 = fmaf((float)c0.x, xv[0], a0);
+      a1 = fmaf((float)c1.x, xv[1], a1);
+      a0 = fmaf((float)c2.x, xv[2], a0);
+      a1 = fmaf((float)c3.x, xv[3], a1);
+      a0 = fmaf((float)c0.y, xv[4], a0);
+      a1 = fmaf((float)c1.y, xv[5], a1);
+      a0 = fmaf((float)c2.y, xv[6], a0);
+      a1 = fmaf((float)c3.y, xv[7], a1);
+    } else {
+      constexpr uint32_t flip = ENC == EG_ENC_SIGNED ? 0x64806480u : 0x64006400u;
+      const half2v c0 = halves((d & 0x00FF00FFu) ^ flip) + zl, c1 = halves((d8 & 0x00FF00FFu) ^ flip) + zl;
+      const float* xv = x + 4 * i;
+      a0 = fmaf((float)c0.x, xv[0], a0);
+      a1 = fmaf((float)c1.x, xv[1], a1);
+      a0 = fmaf((float)c0.y, xv[2], a0);
+      a1 = fmaf((float)c1.y, xv[3], a1);
+    }
+  }
+  return a0 + a1;
+}
+
+// Rows longer than the 256 chunks whose x fits a wave's registers (K over 8192 for int4, 4096 for int8 -
+// the down projection of wider models), up to kLongMaxK: one wave per U rows, x in LDS. A workgroup of
+// 8 waves stages x once - chunk-transposed (x_slot), each chunk's block index beside it - and its waves
+// walk their rows 64 chunks at a time (slots: lane l on chunk l + 64 j), kLongDepth slots' codes in
+// flight; a slot's x is read from LDS once for the U rows. Memory-bound: the codes and scales cross
+// once; the LDS reads are 128 / U bytes per 16 of codes. Against the per-element fallback (a byte load
+// and a divide per code) 4096 x 11008 int4, ref format: 133.6 -> 11.3 us on MI355X.
+constexpr uint32_t kLongMaxK = 15360;  // x and its block indices within 64 KiB of LDS
+constexpr int kLongWaves = 8;
+constexpr int kLongDepth = 4;
+
+template <int BITS, int ENC, int U>
+__global__ __launch_bounds__(64 * kLongWaves) void gemv_long_kernel(
+    const float* __restrict__ x, const uint32_t* packed, const float* scales, const uint32_t* zeros,
+    const float* __restrict__ bias, float* __restrict__ out, uint32_t n, uint32_t chunks, uint32_t chunks_per_block,
+    uint32_t blocks_per_row) {
+  using C = Codes<BITS>;
+  constexpr uint32_t EPC = C::kPerChunk, P = EPC / 4;
+  extern __shared__ __align__(16) uint8_t smem[];
+  float4* const xs = reinterpret_cast<float4*>(smem);                            // chunks * P
+  uint32_t* const blk = reinterpret_cast<uint32_t*>(xs + (size_t)chunks * P);  // chunks
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * kLongWaves + (tid >> 6));
+  const uint32_t waves = gridDim.x * kLongWaves;
+  const uint32_t groups = (n + U - 1) / U, slots = (chunks + 63) / 64;
+  // this wave's row groups: wave, wave + waves, ...; every (group, slot) pair one step
+  const uint32_t mine = wave < groups ? (groups - wave + waves - 1) / waves : 0u, steps = mine * slots;
+  const auto wb = egd::buffer(packed, n * chunks * 16u), sb = egd::buffer(scales, n * blocks_per_row * 4u);
+  const auto zb = egd::buffer(zeros, ((n * blocks_per_row + C::kZeroPerWord - 1) / C::kZeroPerWord) * 4u);
+  struct Step {
+    egd::u32x4 q[U];
+    float s[U];
+    uint32_t zw[U];
+  };
+  // step i's codes (its scales wait for the block indices, so they are loaded by `scales_of`)
+  auto codes_of = [&](uint32_t group, uint32_t slot, Step& t) {
+    const uint32_t c = slot * 64u + lane;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const uint32_t row = group * U + u;
+      const bool in = row < n && c < chunks;
+      t.q[u] = egd::load_b128_nt(wb, in ? (row * chunks + c) * 16u : 0xFFFFFFF0u);
+    }
+  };
+  auto scales_of = [&](uint32_t group, uint32_t slot, Step& t) {
+    const uint32_t c = slot * 64u + lane, b = blk[c < chunks ? c : 0u];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const uint32_t row = group * U + u, i = row * blocks_per_row + b;
+      const bool in = row < n && c < chunks;
+      t.s[u] = egd::load_f32_nt(sb, in ? i * 4u : 0xFFFFFFF0u);
+      if (ENC == EG_ENC_OFFSET_ZEROS) t.zw[u] = egd::load_b32(zb, in ? i / C::kZeroPerWord * 4u : 0xFFFFFFF0u);
+    }
+  };
+  // the next step to load: its group and slot
+  uint32_t lg = wave, ls = 0;
+  auto advance = [&]() {
+    if (++ls == slots) {
+      ls = 0;
+      lg += waves;
+    }
+  };
+  Step st[kLongDepth];
+  const uint32_t g0 = lg;
+#pragma unroll
+  for (int d = 0; d < kLongDepth; d++) {
+    codes_of(lg, ls, st[d]);
+    advance();
+  }
+  // x: coalesced 16-byte reads, transposed on the way (int4: odd elements / 16)
+  constexpr float kOdd = BITS == 4 ? 0.0625f : 1.0f;
+  for (uint32_t i = tid; i < chunks * P; i += blockDim.x) {
+    float4 v = reinterpret_cast<const float4*>(x)[i];
+    v.y *= kOdd;
+    v.w *= kOdd;
+    xs[x_slot<P>(i, chunks)] = v;
+  }
+  for (uint32_t c = tid; c < chunks; c += blockDim.x) blk[c] = c / chunks_per_block;
+  __syncthreads();
+  lg = g0;
+  ls = 0;
+#pragma unroll
+  for (int d = 0; d < kLongDepth; d++) {
+    scales_of(lg, ls, st[d]);
+    advance();
+  }
+  uint32_t cg = wave, cs = 0;
+  float acc[U] = {};
+  for (uint32_t i = 0; i < steps; i += kLongDepth) {
+#pragma unroll
+    for (int d = 0; d < kLongDepth; d++) {
+      if (i + d < steps) {  // wave-uniform
+        const uint32_t c = cs * 64u + lane, cc = c < chunks ? c : 0u;
+        float xr[EPC];
+#pragma unroll
+        for (uint32_t e = 0; e < P; e++) {
+          const float4 v = xs[e * chunks + cc];
+          xr[4 * e] = v.x;
+          xr[4 * e + 1] = v.y;
+          xr[4 * e + 2] = v.z;
+          xr[4 * e + 3] = v.w;
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          uint32_t z = 1u << (BITS - 1);
+          if (ENC == EG_ENC_OFFSET_ZEROS) {
+            const uint32_t b = (cg * U + u) * blocks_per_row + blk[cc];
+            z = (st[d].zw[u] >> (BITS * (b % C::kZeroPerWord))) & ((1u << BITS) - 1u);
+          }
+          const float v = fmaf(st[d].s[u], exact_dot<BITS, ENC>(st[d].q[u], xr, z), acc[u]);
+          acc[u] = c < chunks ? v : acc[u];  // (a slot past the row holds zeros, times x[0..])
+        }
+        if (++cs == slots) {
+#pragma unroll
+          for (int u = 0; u < U; u++) {
+            const uint32_t row = cg * U + u;
+            const float v = egd::team_allsum<64>(acc[u]);
+            if (lane == 0 && row < n) out[row] = bias ? v + bias[row] : v;
+            acc[u] = 0.f;
+          }
+          cs = 0;
+          cg += waves;
+        }
+        codes_of(lg, ls, st[d]);
+        scales_of(lg, ls, st[d]);
+        advance();
+      }
+    }
+  }
+}
+
+using LongFn = void (*)(const float*, const uint32_t*, const float*, const uint32_t*, const float*, float*, uint32_t,
+                        uint32_t, uint32_t, uint32_t);
+
+template <int U>
+LongFn pick_long(int bits, int enc) {
+  if (bits == 4) return enc == EG_ENC_SIGNED ? gemv_long_kernel<4, EG_ENC_SIGNED, U> : gemv_long_kernel<4, EG_ENC_OFFSET_ZEROS, U>;
+  return enc == EG_ENC_SIGNED ? gemv_long_kernel<8, EG_ENC_SIGNED, U> : gemv_long_kernel<8, EG_ENC_OFFSET_ZEROS, U>;
+}
+
 // The LM head over an f16 (BITS 16) or f32 (BITS 32) tied table (the 'f16' / 'f32' dtypes of
 // embedding_variants.ts:46-74, 135-180): out[n] = sum_k x[k] table[n][k]. With no codes to
 // unpack the launch streams the table: one wave per row, two rows per step (their loads issued
@@ -570,6 +751,16 @@ int launch(eg_context* ctx, const QuantView& v) {
     if ((st = partials_fit(grid)) != EG_OK) return st;
     a.stamp = eg::stamp_slot(ctx);
     hipLaunchKernelGGL(fn, dim3(grid), dim3(256), smem, ctx->stream, a);
+  } else if (mode == kPlain && !fused && aligned && v.k % epc == 0 && v.block_size % epc == 0 && chunks > 256 &&
+             v.k <= kLongMaxK) {
+    // one row per wave while they all fit on the device at once (two workgroups per CU), else two
+    const uint64_t resident = (uint64_t)ctx->cu_count * 2;
+    const bool two = v.n > resident * kLongWaves;
+    const uint64_t groups = two ? ((uint64_t)v.n + 1) / 2 : v.n;
+    grid = (uint32_t)std::min<uint64_t>(resident, (groups + kLongWaves - 1) / kLongWaves);
+    const LongFn fn = two ? pick_long<2>(v.bits, v.encoding) : pick_long<1>(v.bits, v.encoding);
+    hipLaunchKernelGGL(fn, dim3(grid), dim3(64 * kLongWaves), v.k * 4u + chunks * 4u, ctx->stream, v.x, v.packed, v.scales,
+                       v.zeros, v.bias, v.out + v.out_offset, v.n, chunks, v.block_size / epc, v.blocks_per_row);
   } else {
     uint64_t blocks = (v.n + kWaves - 1) / kWaves;
     const uint64_t cap = (uint64_t)ctx->cu_count * 8;
