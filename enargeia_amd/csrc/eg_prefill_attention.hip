@@ -21,8 +21,7 @@
 //      workspace and 3. a combine launch merges the splits in split order.
 //
 // The f32 cache variant (eg_attention_prefill_f32; cache_variants.ts:21-40 generates the same
-// kernels per cache dtype) appends exact f32 rows and runs the attention as f32 FMAs: the
-// matrix cores here take f16 or bf16 operands, which would round the f32 keys and values.
+// kernels per cache dtype) appends exact f32 rows and runs the attention on the f32 matrix cores.
 #include <algorithm>
 #include <type_traits>
 
@@ -32,6 +31,7 @@ namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // 16 bytes at any float's address
 
 constexpr int kD = 64;           // head_dim (the path's models)
 constexpr int kQ = 64;           // queries per workgroup
@@ -80,105 +80,6 @@ __global__ __launch_bounds__(256) void rope_append_kernel(const float* __restric
   }
   for (uint32_t p = tid; p < d.kv_heads * kD; p += blockDim.x)
     v_cache[(size_t)pos * d.kv_heads * kD + p] = to_cache<CT>(v[(size_t)i * d.kv_heads * kD + p]);
-}
-
-// The attention over an f32 cache. One workgroup per (query row i, kv head): the group's query
-// heads (at most kF32Group) walk the keys [0, query_begin + i] in tiles of 256, one key per
-// thread - its scores, products summed in element order - with the online softmax in f32 (the
-// tile's max and sum of exp per head by fixed-order wave and cross-wave reductions), then each
-// thread's outputs (head g, element e; two per thread) take the tile's weighted V rows in key
-// order. Keys past the query's limit weigh 0, as the reference's NEG_LARGE mask makes them.
-constexpr uint32_t kF32Tile = 256;
-constexpr uint32_t kF32Group = 8;
-
-__global__ __launch_bounds__(256) void attention_f32_kernel(const float* __restrict__ q_rope,
-                                                            const float* __restrict__ k_cache,
-                                                            const float* __restrict__ v_cache, float* __restrict__ out,
-                                                            eg_attention_prefill_dims d) {
-  __shared__ __attribute__((aligned(16))) float qs[kF32Group][kD];
-  __shared__ float pw[kF32Group][kF32Tile];  // the tile's weights e^(s - M)
-  __shared__ float red[4][kF32Group];        // per-wave maxima, then sums
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  const uint32_t i = blockIdx.x, kv = blockIdx.y;
-  const uint32_t G = d.heads / d.kv_heads, h0 = kv * G;
-  const uint32_t limit = d.query_begin + i;  // the last key this query sees
-  for (uint32_t t = tid; t < G * kD; t += blockDim.x) qs[t / kD][t % kD] = q_rope[((size_t)i * d.heads + h0) * kD + t];
-  __syncthreads();
-  float M[kF32Group], L[kF32Group];  // running max and sum per head (the same in every thread)
-#pragma unroll
-  for (uint32_t g = 0; g < kF32Group; g++) {
-    M[g] = -INFINITY;
-    L[g] = 0.f;
-  }
-  // this thread's outputs: (g, e) = (tid / 64, tid % 64) and (4 + tid / 64, tid % 64)
-  const uint32_t e = lane, ga = wave, gb = wave + 4;
-  float acc_a = 0.f, acc_b = 0.f;
-  const size_t row_pitch = (size_t)d.kv_heads * kD;
-  for (uint32_t t0 = 0; t0 <= limit; t0 += kF32Tile) {
-    const uint32_t key = t0 + tid;
-    const bool valid = key <= limit;
-    float s[kF32Group];
-    {
-      float4 kr[kD / 4];
-      const float4* src = reinterpret_cast<const float4*>(k_cache + (valid ? key : 0) * row_pitch + kv * kD);
-#pragma unroll
-      for (int w = 0; w < kD / 4; w++) kr[w] = src[w];
-#pragma unroll
-      for (uint32_t g = 0; g < kF32Group; g++) {
-        float a = 0.f;
-        if (g < G) {
-#pragma unroll
-          for (int w = 0; w < kD / 4; w++) {
-            const float4 qv = *reinterpret_cast<const float4*>(&qs[g][4 * w]);
-            a = fmaf(qv.x, kr[w].x, a);
-            a = fmaf(qv.y, kr[w].y, a);
-            a = fmaf(qv.z, kr[w].z, a);
-            a = fmaf(qv.w, kr[w].w, a);
-          }
-        }
-        s[g] = valid ? a : -INFINITY;
-      }
-    }
-    // the tile's max per head, then the new running max and the rescale of what came before
-    float scale[kF32Group];
-#pragma unroll
-    for (uint32_t g = 0; g < kF32Group; g++) {
-      const float m = egd::team_allmax<64>(s[g]);
-      if (lane == 0) red[wave][g] = m;
-    }
-    __syncthreads();
-#pragma unroll
-    for (uint32_t g = 0; g < kF32Group; g++) {
-      const float mt = fmaxf(fmaxf(red[0][g], red[1][g]), fmaxf(red[2][g], red[3][g]));
-      const float mn = fmaxf(M[g], mt);
-      scale[g] = g < G ? expf(M[g] - mn) : 0.f;  // e^-inf = 0 on the first tile
-      M[g] = mn;
-    }
-    __syncthreads();  // red is reused below
-#pragma unroll
-    for (uint32_t g = 0; g < kF32Group; g++) {
-      const float p = valid && g < G ? expf(s[g] - M[g]) : 0.f;
-      pw[g][tid] = p;
-      const float sum = egd::team_allsum<64>(p);
-      if (lane == 0) red[wave][g] = sum;
-    }
-    __syncthreads();
-#pragma unroll
-    for (uint32_t g = 0; g < kF32Group; g++) L[g] = fmaf(L[g], scale[g], ((red[0][g] + red[1][g]) + red[2][g]) + red[3][g]);
-    const uint32_t n = min(kF32Tile, limit + 1 - t0);
-    const float* vrow = v_cache + (size_t)t0 * row_pitch + kv * kD + e;
-    float sa = 0.f, sb = 0.f;
-    for (uint32_t j = 0; j < n; j++) {
-      const float vv = vrow[(size_t)j * row_pitch];
-      sa = fmaf(pw[ga][j], vv, sa);
-      sb = fmaf(pw[gb][j], vv, sb);
-    }
-    acc_a = fmaf(acc_a, scale[ga], sa);
-    acc_b = fmaf(acc_b, scale[gb], sb);
-    __syncthreads();  // pw and red are rewritten by the next tile
-  }
-  if (ga < G) out[((size_t)i * d.heads + h0 + ga) * kD + e] = acc_a / L[ga];
-  if (gb < G) out[((size_t)i * d.heads + h0 + gb) * kD + e] = acc_b / L[gb];
 }
 
 // Split partials: o [split][query][head][kD] (unnormalised), then m and l [split][query][head].
@@ -410,8 +311,215 @@ __global__ __launch_bounds__(256) void attention_kernel(const float* __restrict_
   }
 }
 
+// ---- the f32 cache --------------------------------------------------------------------------
+//
+// The attention over f32 rows on the f32 matrix cores (v_mfma_f32_16x16x4_f32: f32 operands, products
+// and sums), in attention_kernel's transposed form: S^T = K Q^T, O^T += V^T P^T, 16 queries per wave, 64
+// per workgroup, key tiles of 64, the same online softmax and key splits. The operand layouts hold one
+// k value per lane and step, and k is taken in the order that keeps every LDS read 16 bytes wide:
+//   S^T block n (keys 16 n + lr): lane group g owns d = 16 g .. +16, four reads per key;
+//   O^T: step (n, e) multiplies key 16 n + 4 g + e, which is where the S^T accumulators hold it, so P goes
+//   from them straight into the operand; block nd's row lr is d = 4 lr + nd, one read per key for all four
+//   blocks, and a lane's o[0..3][e] are the four consecutive d = 16 g + 4 e .. +4.
+// K and V rows go from memory to LDS directly, the next tile's while this one is multiplied; K's 16-byte
+// slots are swizzled by the row. Sums stay short for their error's sake: a score is two chains of 32 products,
+// a tile's values are summed by themselves before they are added. MFMA-bound: 128 of 32 cycles per wave and tile. Against a workgroup per
+// query row with f32 FMAs: 256 queries at keys up to 2048, 14 / 2 heads, 208.7 -> 35.2 us on MI355X (RoPE,
+// append and combine included).
+constexpr uint32_t kF32Group = 8;  // query heads per kv head
+constexpr uint32_t kF32Tile = kK * kD * 4;  // bytes of a K (or V) tile
+
+__global__ __launch_bounds__(256) void attention_f32_kernel(const float* __restrict__ q_rope,
+                                                            const float* __restrict__ k_cache,
+                                                            const float* __restrict__ v_cache, float* __restrict__ out,
+                                                            eg_attention_prefill_dims d, Splits sp) {
+  __shared__ __attribute__((aligned(16))) uint8_t Ks[2][kF32Tile];
+  __shared__ __attribute__((aligned(16))) uint8_t Vs[2][kF32Tile];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t lr = lane & 15u, lg = lane >> 4;
+  const uint32_t h = blockIdx.y, kv = h / (d.heads / d.kv_heads);
+  const uint32_t q0 = (gridDim.x - 1 - blockIdx.x) * kQ;  // the longest causal walks first
+  const uint32_t query = q0 + wave * 16 + lr;
+
+  float qb[16];
+  {
+    const bool in = query < d.queries;
+    const float4* src = reinterpret_cast<const float4*>(q_rope + ((size_t)(in ? query : 0) * d.heads + h) * kD + 16 * lg);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const float4 v = in ? src[j] : make_float4(0.f, 0.f, 0.f, 0.f);
+      qb[4 * j] = v.x;
+      qb[4 * j + 1] = v.y;
+      qb[4 * j + 2] = v.z;
+      qb[4 * j + 3] = v.w;
+    }
+  }
+  f32x4 o[4];
+#pragma unroll
+  for (int n = 0; n < 4; n++) o[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+
+  const uint32_t last_query = min(q0 + (uint32_t)kQ, d.queries) - 1;
+  uint32_t key_end = d.query_begin + last_query + 1, key_begin = 0;
+  if (sp.o) {
+    key_begin = blockIdx.z * sp.keys;
+    key_end = min(key_end, key_begin + sp.keys);
+  }
+  const uint32_t ntiles = key_end > key_begin ? (key_end - key_begin + kK - 1) / kK : 0;
+  const uint32_t limit = d.query_begin + query;
+  const uint32_t open_end = min(d.query_begin + q0 + wave * 16 + 1, key_end);
+
+  // A tile's rows, 4 per load of 1 KiB: row r's 16-byte slot j of K at LDS slot j ^ (r % 16), of V at j.
+  // Rows past the last key repeat it (its scores are masked).
+  const size_t pitch = (size_t)d.kv_heads * kD;
+  auto load_tile = [&](uint32_t j0, uint32_t buf) {
+    const auto kr = egd::buffer(k_cache + (size_t)j0 * pitch, min(key_end - j0, (uint32_t)kK) * d.kv_heads * (kD * 4u));
+    const auto vr = egd::buffer(v_cache + (size_t)j0 * pitch, min(key_end - j0, (uint32_t)kK) * d.kv_heads * (kD * 4u));
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) {
+      const uint32_t r = (4 * i + wave) * 4 + lg, row = min(r, key_end - j0 - 1);
+      const uint32_t at = (row * d.kv_heads + kv) * (kD * 4u);
+      egd::load_to_lds(kr, Ks[buf] + (4 * i + wave) * 1024u, at + 16u * (lr ^ (r & 15u)));
+      egd::load_to_lds(vr, Vs[buf] + (4 * i + wave) * 1024u, at + 16u * lr);
+    }
+  };
+  auto settle = [&]() {
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt 0: the memory-to-LDS loads have landed
+    __syncthreads();
+  };
+  if (ntiles) load_tile(key_begin, 0);
+  settle();
+  for (uint32_t t = 0; t < ntiles; t++) {
+    const uint32_t j0 = key_begin + t * kK, buf = t & 1u;
+    // (the other buffer was last read before the barrier that ended the previous tile)
+    if (t + 1 < ntiles) load_tile(j0 + kK, buf ^ 1u);
+
+    f32x4 s[4], s1[4];
+#pragma unroll
+    for (int n = 0; n < 4; n++) s[n] = s1[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (uint32_t j = 0; j < 4; j++) {
+      f32x4 ka[4];
+#pragma unroll
+      for (uint32_t n = 0; n < 4; n++)
+        ka[n] = *reinterpret_cast<const f32x4*>(Ks[buf] + (16 * n + lr) * (kD * 4u) + 16u * ((4 * lg + j) ^ lr));
+#pragma unroll
+      for (int c = 0; c < 4; c++)
+#pragma unroll
+        for (int n = 0; n < 4; n++) {
+          f32x4& half = j < 2 ? s[n] : s1[n];
+          half = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[n][c], qb[4 * j + c], half, 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < 4; n++) s[n] += s1[n];
+
+    const bool masked = j0 + kK > open_end;
+    if (masked) {
+#pragma unroll
+      for (int n = 0; n < 4; n++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const uint32_t j = j0 + 16 * n + 4 * lg + e;
+          if (!(j <= limit && j < key_end)) s[n][e] = -INFINITY;
+        }
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int n = 0; n < 4; n++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) mx = fmaxf(mx, s[n][e]);
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float mnew = fmaxf(m, mx);
+    // (no visible key yet: nothing is kept, and no infinity is taken from another)
+    const float base = mnew == -INFINITY ? 0.f : mnew;
+    const float alpha = mnew == -INFINITY ? 1.f : expf(m - base);
+    float sum = 0.f;
+#pragma unroll
+    for (int n = 0; n < 4; n++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const float p = expf(s[n][e] - base);
+        s[n][e] = p;
+        sum += p;
+      }
+    l = fmaf(l, alpha, sum);
+    m = mnew;
+
+    // In a masked tile a key's weight of 0 must drop its value even where that is infinite or NaN (a
+    // later row of the chunk): if any is, the tile's values are added one visible key at a time.
+    f32x4 ot[4];
+#pragma unroll
+    for (int n = 0; n < 4; n++) ot[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    bool plain = true;
+    if (masked) {
+      bool finite = true;
+#pragma unroll
+      for (uint32_t n = 0; n < 16; n++) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(Vs[buf] + (4 * n + lg) * (kD * 4u) + 16u * lr);
+#pragma unroll
+        for (int c = 0; c < 4; c++) finite = finite && isfinite(v[c]);
+      }
+      plain = __builtin_amdgcn_ballot_w64(!finite) == 0;
+    }
+    if (plain) {
+#pragma unroll
+      for (int n = 0; n < 4; n++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const f32x4 va = *reinterpret_cast<const f32x4*>(Vs[buf] + (16 * n + 4 * lg + e) * (kD * 4u) + 16u * lr);
+#pragma unroll
+          for (int nd = 0; nd < 4; nd++) ot[nd] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[nd], s[n][e], ot[nd], 0, 0, 0);
+        }
+    } else {
+#pragma unroll
+      for (uint32_t n = 0; n < 4; n++)
+#pragma unroll
+        for (uint32_t e = 0; e < 4; e++)
+          for (uint32_t g = 0; g < 4; g++) {
+            const uint32_t key = 16 * n + 4 * g + e;
+            const float p = __shfl(s[n][e], lr + 16 * g, 64);
+            if (j0 + key > limit || j0 + key >= key_end) continue;
+#pragma unroll
+            for (uint32_t c = 0; c < 4; c++) {
+              const f32x4 v = *reinterpret_cast<const f32x4*>(Vs[buf] + key * (kD * 4u) + 16u * (4 * lg + c));
+#pragma unroll
+              for (int nd = 0; nd < 4; nd++) ot[nd][c] = fmaf(p, v[nd], ot[nd][c]);
+            }
+          }
+    }
+#pragma unroll
+    for (int n = 0; n < 4; n++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) o[n][e] = fmaf(o[n][e], alpha, ot[n][e]);
+    settle();
+  }
+
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (query >= d.queries) return;
+  if (sp.o) {
+    const size_t row = ((size_t)blockIdx.z * d.queries + query) * d.heads + h;
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      *reinterpret_cast<float4*>(&sp.o[row * kD + 16 * lg + 4 * e]) = make_float4(o[0][e], o[1][e], o[2][e], o[3][e]);
+    if (lg == 0) {
+      float* mlp = sp.o + (size_t)sp.count * d.queries * d.heads * kD;
+      mlp[row] = m;
+      mlp[(size_t)sp.count * d.queries * d.heads + row] = l;
+    }
+    return;
+  }
+  float* dst = out + ((size_t)query * d.heads + h) * kD + 16 * lg;
+#pragma unroll
+  for (int e = 0; e < 4; e++)
+    *reinterpret_cast<f32x4u*>(dst + 4 * e) = f32x4u{o[0][e] / l, o[1][e] / l, o[2][e] / l, o[3][e] / l};
+}
+
 // The splits merged: out = sum_z o_z e^(m_z - M) / sum_z l_z e^(m_z - M), M = max_z m_z, splits
-// in order (an empty split has m = NEG_LARGE and l = 0, weight 0). One thread per 4 elements of a
+// in order (an empty split has l = 0 and is left out). One thread per 4 elements of a
 // row. A row's splits past its causal limit are empty (z > zmax: the split's first key is past the
 // row's last) and are not read. Up to kFastSplits splits, the statistics and values of the
 // others are loaded at once (no chain of dependent round trips); more splits take the loop. Both
@@ -420,7 +528,7 @@ constexpr uint32_t kFastSplits = 8;
 
 __device__ __forceinline__ float4 merged(const float* __restrict__ part, const float* m, const float* l, size_t total,
                                          uint32_t rows, size_t row, size_t idx, uint32_t splits, uint32_t zmax) {
-  float M = kMasked, L = 0.f;
+  float M = -INFINITY, L = 0.f;
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
   if (splits <= kFastSplits) {
     float mz[kFastSplits], lz[kFastSplits];
@@ -438,7 +546,7 @@ __device__ __forceinline__ float4 merged(const float* __restrict__ part, const f
       if (z <= zmax) M = fmaxf(M, mz[z]);
 #pragma unroll
     for (uint32_t z = 0; z < kFastSplits; z++) {
-      if (z <= zmax && lz[z] > 0.f) {
+      if (z <= zmax && lz[z] != 0.f) {  // (a NaN sum stays in)
         const float w = expf(mz[z] - M);
         L = fmaf(lz[z], w, L);
         acc.x = fmaf(vz[z].x, w, acc.x);
@@ -451,7 +559,7 @@ __device__ __forceinline__ float4 merged(const float* __restrict__ part, const f
     for (uint32_t z = 0; z <= zmax; z++) M = fmaxf(M, m[(size_t)z * rows + row]);
     for (uint32_t z = 0; z <= zmax; z++) {
       const float lzz = l[(size_t)z * rows + row];
-      if (!(lzz > 0.f)) continue;
+      if (lzz == 0.f) continue;
       const float w = expf(m[(size_t)z * rows + row] - M);
       L = fmaf(lzz, w, L);
       const float4 v = reinterpret_cast<const float4*>(part + (size_t)z * total)[idx];
@@ -475,7 +583,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ 
     const uint32_t zmax = min(splits - 1, (query_begin + (uint32_t)(row / heads)) / split_keys);
     const float4 v = merged(part, m, l, total, rows, row, idx, splits, zmax);
     if (out_bf16) reinterpret_cast<uint2*>(out)[idx] = make_uint2(egd::pack_bf16(v.x, v.y), egd::pack_bf16(v.z, v.w));
-    else reinterpret_cast<float4*>(out)[idx] = v;
+    else *reinterpret_cast<f32x4u*>(out + 4 * idx) = f32x4u{v.x, v.y, v.z, v.w};
   }
 }
 
@@ -503,24 +611,21 @@ int eg::check_attention_prefill(eg_context* ctx, const char* op, const eg_attent
   return EG_OK;
 }
 
-int eg::attention_prefill_run(eg_context* ctx, const float* q_rope, const uint16_t* k_cache, const uint16_t* v_cache,
-                              float* out, const eg_attention_prefill_dims& d, bool out_bf16) {
-  const char* op = "attention_prefill";
-  if ((reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache)) & 15u)
-    return eg::fail(ctx, EG_ERR_INVALID, "%s: the caches must be 16-byte aligned", op);
-  if ((reinterpret_cast<uintptr_t>(q_rope) | reinterpret_cast<uintptr_t>(out)) & 15u)
-    return eg::fail(ctx, EG_ERR_INVALID, "%s: q_rope and out must be 16-byte aligned", op);
-  if (d.queries == 0) return EG_OK;
-  // Keys split over a long key range, within the workspace: where the (query block, head) grid
-  // leaves most CUs idle, into splits of at least 4 key tiles, about one workgroup per CU in all;
-  // and so that no workgroup walks more than 8 tiles - the causal limit makes the last query
-  // blocks of a long chunk the longest, and with the split their keys spread over more
-  // workgroups while the early blocks' later splits are empty.
+namespace {
+
+// Keys split over a long key range, within the workspace: where the (query block, head) grid
+// leaves most CUs idle, into splits of at least 4 key tiles, about per_cu workgroups per CU in all
+// (2 over an f32 cache, whose time is the longest CU's MFMAs: 256 queries at 1792 take 4 us
+// more at 1; f16 rows, bound by latency, take 19.3 us at 1 and 19.8 at 2);
+// and so that no workgroup walks more than 8 tiles - the causal limit makes the last query
+// blocks of a long chunk the longest, and with the split their keys spread over more
+// workgroups while the early blocks' later splits are empty.
+Splits splits_for(eg_context* ctx, const eg_attention_prefill_dims& d, uint32_t per_cu = 1) {
   const uint32_t blocks = (d.queries + kQ - 1) / kQ;
   const uint64_t grid = (uint64_t)blocks * d.heads;
   const uint32_t tiles = (d.keys + kK - 1) / kK;
   const uint32_t cap = ctx->attention_split_tiles;
-  const uint64_t target = (uint64_t)ctx->cu_count * ctx->attention_split_fill;
+  const uint64_t target = (uint64_t)ctx->cu_count * ctx->attention_split_fill * per_cu;
   uint32_t splits = 1;
   if (tiles >= 8) {
     if (grid < target) splits = (uint32_t)std::min<uint64_t>((target + grid - 1) / grid, tiles / 4);
@@ -534,6 +639,22 @@ int eg::attention_prefill_run(eg_context* ctx, const float* q_rope, const uint16
     sp.count = (d.keys + sp.keys - 1) / sp.keys;
     sp.o = reinterpret_cast<float*>(eg::partials(ctx));
   }
+  return sp;
+}
+
+}  // namespace
+
+int eg::attention_prefill_run(eg_context* ctx, const float* q_rope, const uint16_t* k_cache, const uint16_t* v_cache,
+                              float* out, const eg_attention_prefill_dims& d, bool out_bf16) {
+  const char* op = "attention_prefill";
+  if ((reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache)) & 15u)
+    return eg::fail(ctx, EG_ERR_INVALID, "%s: the caches must be 16-byte aligned", op);
+  if ((reinterpret_cast<uintptr_t>(q_rope) | reinterpret_cast<uintptr_t>(out)) & 15u)
+    return eg::fail(ctx, EG_ERR_INVALID, "%s: q_rope and out must be 16-byte aligned", op);
+  if (d.queries == 0) return EG_OK;
+  const uint32_t blocks = (d.queries + kQ - 1) / kQ;
+  const uint64_t rows = (uint64_t)d.queries * d.heads;
+  const Splits sp = splits_for(ctx, d);
   hipLaunchKernelGGL(attention_kernel, dim3(blocks, d.heads, sp.count), dim3(256), 0, ctx->stream, q_rope, k_cache,
                      v_cache, out, d, sp, out_bf16 ? 1u : 0u);
   if (sp.o) {
@@ -583,7 +704,15 @@ extern "C" int eg_attention_prefill_f32(eg_context* ctx, const float* q, const f
     return eg::fail(ctx, EG_ERR_INVALID, "%s: the caches and q_rope must be 16-byte aligned", op);
   hipLaunchKernelGGL(rope_append_kernel<float>, dim3(d.queries), dim3(256), 0, ctx->stream, q, k, v, q_rope, k_cache,
                      v_cache, d);
-  hipLaunchKernelGGL(attention_f32_kernel, dim3(d.queries, d.kv_heads), dim3(256), 0, ctx->stream, q_rope, k_cache,
-                     v_cache, out, d);
+  const uint32_t blocks = (d.queries + kQ - 1) / kQ;
+  const uint64_t rows = (uint64_t)d.queries * d.heads;
+  const Splits sp = splits_for(ctx, d, 2);
+  hipLaunchKernelGGL(attention_f32_kernel, dim3(blocks, d.heads, sp.count), dim3(256), 0, ctx->stream, q_rope, k_cache,
+                     v_cache, out, d, sp);
+  if (sp.o) {
+    const uint32_t cblocks = (uint32_t)std::min<uint64_t>((rows * kD / 4 + 255) / 256, (uint64_t)ctx->cu_count * 8);
+    hipLaunchKernelGGL(combine_kernel, dim3(cblocks), dim3(256), 0, ctx->stream, sp.o, out, (uint32_t)rows, sp.count, 0u,
+                       d.heads, d.query_begin, sp.keys);
+  }
   return eg::check_launch(ctx, op);
 }

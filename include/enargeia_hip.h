@@ -148,7 +148,7 @@ EG_API int eg_matmul_q4_decode(eg_context* ctx, const float* x, const uint32_t* 
 /* matmul_q4_prefill (matmul_q4_prefill.wgsl:77-162): for m rows of x,
  *   out[r*out_stride + col + out_offset] = sum_k x[r,k] * W[col,k] (+ bias[col])
  * on the matrix cores: x and the dequantized weights are rounded to bf16, products are
- * accumulated in f32 (gfx950 v_mfma_f32_16x16x32_bf16). Same weight streams as decode. */
+ * accumulated in f32 (gfx950 v_mfma_f32_32x32x16_bf16). Same weight streams as decode. */
 EG_API int eg_matmul_q4_prefill(eg_context* ctx, const float* x, const uint32_t* packed,
                          const float* scales, const uint32_t* zeros, const float* bias,
                          float* out, const eg_matmul_q4_dims* dims, int encoding, int bits);
@@ -510,8 +510,9 @@ EG_API int eg_attention_prefill(eg_context* ctx, const float* q, const float* k,
                                 uint16_t* v_cache, float* q_rope, float* out,
                                 const eg_attention_prefill_dims* dims);
 /* eg_attention_prefill over caches of f32 rows (cache_variants.ts:21-40 and 81-145 for the f32
- * dtype): the rotated k and v rows are appended exactly and the attention runs on f32 FMAs
- * with f32 operands throughout; at most 8 query heads per kv head. */
+ * dtype): the rotated k and v rows are appended exactly and the attention runs on the f32 matrix
+ * cores (v_mfma_f32_16x16x4_f32) with f32 operands throughout, over a long key range in splits that
+ * meet in the context's workspace; at most 8 query heads per kv head. */
 EG_API int eg_attention_prefill_f32(eg_context* ctx, const float* q, const float* k, const float* v, float* k_cache,
                                     float* v_cache, float* q_rope, float* out,
                                     const eg_attention_prefill_dims* dims);
