@@ -416,6 +416,13 @@ __device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t r, void* lds,
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, offset, 0, 0, 0);
 }
 
+// A 4 x 16 block of 16-bit values read from LDS transposed, per group of 16 lanes: lane i of the group points
+// at 4 values of row i / 4 (columns 4 (i % 4) .. +4) and receives column i of the 4 rows.
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ s16x4 lds_read_transposed(const void* lds) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)lds);
+}
+
 // The same accesses with an explicit cache policy: AUX = 0 is the default policy; AUX = kCoherent
 // (sc1) is the agent-scope coherent form egd::put / egd::get use, for data another workgroup of
 // the same launch writes or reads.

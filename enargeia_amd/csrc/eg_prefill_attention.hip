@@ -10,7 +10,7 @@
 //      path), q pre-scaled by 1/sqrt(D) into q_rope, k and v appended to the f16 caches at
 //      positions [query_begin, query_begin + queries).
 //   2. attention: flash attention, one workgroup per (64 queries, head), 16 queries per wave.
-//      Key tiles of 64 are staged through LDS (K row-major, V transposed); S = Q K^T and
+//      Key tiles of 64 are staged through LDS; S = Q K^T and
 //      O += P V run on v_mfma_f32_16x16x32_f16 (f16 operands - the cache is f16 already, q and
 //      the softmax weights are rounded to f16 - with f32 accumulation), the softmax is the
 //      online (running max / sum) form in f32, masked scores are the reference's NEG_LARGE.
@@ -36,7 +36,6 @@ typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // 16 byt
 constexpr int kD = 64;           // head_dim (the path's models)
 constexpr int kQ = 64;           // queries per workgroup
 constexpr int kK = 64;           // keys per tile
-constexpr int kRow = kK + 8;     // LDS row pitch in f16 (16 bytes of padding)
 constexpr float kMasked = -1.0e30f;  // NEG_LARGE, cache_variants.ts
 
 using egd::float_to_half;
@@ -91,75 +90,48 @@ struct Splits {
 
 constexpr float kLog2e = 1.44269504088896340736f;
 
-// One key tile's K and V in registers between its global loads and its LDS stores: K as two
-// 16-byte pieces of key tid / 4 (d 16 * (tid % 4) .. +16), V as 4 d values (4 * (tid % 16) .. +4)
-// of the 4 keys 4 * (tid / 16) .. +4. The caches are read through buffer resources that end at
-// the workgroup's last key: rows past it read as zeros without touching memory (a V row there
-// must be finite - its weight is 0 - and no branch is needed).
-struct KVTile {
-  egd::u32x4 k[2];
-  uint64_t v[4];
-};
-
-struct KVStream {
-  __amdgpu_buffer_rsrc_t k, v;
-  uint32_t koff, voff, pitch;  // this thread's byte offsets in tile 0; bytes between cache rows
-};
-
-__device__ __forceinline__ void load_tile(KVTile& t, const KVStream& st, uint32_t j0) {
-  const uint32_t base = j0 * st.pitch;
-  t.k[0] = egd::load_b128(st.k, st.koff + base);
-  t.k[1] = egd::load_b128(st.k, st.koff + base + 16u);
-#pragma unroll
-  for (int i = 0; i < 4; i++) t.v[i] = egd::load_b64(st.v, st.voff + base + i * st.pitch);
-}
-
-// LDS row of key r in Ks: bit 2 flipped where bit 4 is set, so the 16 rows one S^T operand read
-// touches (keys 0-3, 8-11, 16-19, 24-27 of a half tile, plus 4 for odd blocks) fall in 16
-// different groups of 4 banks.
-__device__ __forceinline__ uint32_t ks_row(uint32_t r) { return r ^ (((r >> 4) & 1u) << 2); }
-
-// K row-major, V transposed: the 4 x 4 block of V (keys 4a .. 4a+3, d c .. c+3) becomes 4 rows of
-// Vt, one 8-byte store each.
-__device__ __forceinline__ void store_tile(const KVTile& t, uint16_t (*Ks)[kRow], uint16_t (*Vt)[kRow], uint32_t tid) {
-  {
-    const uint32_t r = ks_row(tid >> 2), c = (tid & 3u) * 16u;
-    *reinterpret_cast<egd::u32x4*>(&Ks[r][c]) = t.k[0];
-    *reinterpret_cast<egd::u32x4*>(&Ks[r][c + 8]) = t.k[1];
-  }
-  const uint32_t a = tid >> 4, c = (tid & 15u) * 4u;
-  // t.v[i] = (d c, c+1 | c+2, c+3) of key 4a + i; row c + e of Vt takes element e of each key
-#pragma unroll
-  for (int e = 0; e < 4; e++) {
-    const int sh = 32 * (e >> 1);
-    const uint32_t k0 = (uint32_t)(t.v[0] >> sh), k1 = (uint32_t)(t.v[1] >> sh);
-    const uint32_t k2 = (uint32_t)(t.v[2] >> sh), k3 = (uint32_t)(t.v[3] >> sh);
-    // element e is the low (e even) or high (e odd) half of word e / 2
-    const uint2 row = (e & 1) ? make_uint2((k0 >> 16) | (k1 & 0xFFFF0000u), (k2 >> 16) | (k3 & 0xFFFF0000u))
-                              : make_uint2((k0 & 0xFFFFu) | (k1 << 16), (k2 & 0xFFFFu) | (k3 << 16));
-    *reinterpret_cast<uint2*>(&Vt[c + e][4 * a]) = row;
-  }
+// Max over the 4 lanes that hold a query (lr, lr + 16, lr + 32, lr + 48), in the vector units.
+__device__ __forceinline__ float max_of_query(float x) {
+  const uint32_t a = __float_as_uint(x);
+  const auto r = __builtin_amdgcn_permlane32_swap(a, a, false, false);
+  const uint32_t b = __float_as_uint(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
+  const auto t = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+  return fmaxf(__uint_as_float(t[0]), __uint_as_float(t[1]));
 }
 
 // Flash attention in the transposed form: S^T = K Q^T and O^T += V^T P^T, so that each lane holds
 // ONE query's scores (the MFMA D layout puts a column in a lane) and P goes from the S^T
-// accumulators straight into the B operand of the second product, with no LDS round trip.
+// accumulators straight into the B operand of the second product, with no LDS round trip: lane
+// group g = lane / 16 holds keys 16 n + 4 g + e of S^T block n, and its 8 k-slots of the half h of
+// the second product are those of blocks 2 h and 2 h + 1. The V^T operand is two transposed reads
+// of 4 keys each from V as the cache has it.
 //
-// Key order inside a tile: row m = 4g + e of S^T block n (n < 4, g = m / 4, e = m % 4) is key
-// 32 (n / 2) + 8 g + 4 (n % 2) + e, so a lane (column lr, group g = lane / 16) holds, for each half
-// h of the tile, the 8 consecutive keys 32 h + 8 g .. +8 - exactly the 8 k-slots of its P^T operand
-// in the second product, whose V^T operand then reads 8 consecutive keys of a Vt row.
-__global__ __launch_bounds__(256) void attention_kernel(const float* __restrict__ q_rope,
-                                                        const uint16_t* __restrict__ k_cache,
-                                                        const uint16_t* __restrict__ v_cache, float* __restrict__ out,
-                                                        eg_attention_prefill_dims d, Splits sp, uint32_t out_bf16) {
-  __shared__ __attribute__((aligned(16))) uint16_t Ks[2][kK][kRow];  // [buffer][key][d]
-  __shared__ __attribute__((aligned(16))) uint16_t Vt[2][kD][kRow];  // [buffer][d][key]
-  const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
+// K and V rows go from memory to LDS directly (16-byte slots, 8 to a row; the next tile's while
+// this one is multiplied). Row r's slot j is kept at j ^ ((r / 2) % 8) in K, which spreads the 16
+// rows of an operand read over all banks, and at j ^ 2 ((r / 2) % 4) in V, which spreads the 4 rows
+// a lane group's transposed read touches, and those of two groups: no conflicts. (Rows through
+// registers, V transposed on the way into LDS: 62% of the LDS cycles were conflicts, and LDS was the
+// busiest unit.) Bound by the softmax's vector instructions and, with few workgroups, their latency;
+// 32 queries per wave, half the LDS reads, was slower at every size (2048 queries: 28 us for 25).
+// MI355X, 14 heads, this kernel alone: 2048 queries 38.8 -> 24.3 us, 256 at 1792 13.0 -> 10.8.
+constexpr uint32_t kTileBytes = kK * kD * 2;
+
+// (5 waves per SIMD, what LDS holds; the bound also keeps the accumulators out of the AGPRs.)
+__global__ __launch_bounds__(256, 5) void attention_kernel(const float* __restrict__ q_rope,
+                                                           const uint16_t* __restrict__ k_cache,
+                                                           const uint16_t* __restrict__ v_cache,
+                                                           float* __restrict__ out, eg_attention_prefill_dims d,
+                                                           Splits sp, uint32_t out_bf16) {
+  // [buffer][K or V][key][d]. (One array: between two the compiler has a read of K wait for the loads
+  // into the other buffer.)
+  __shared__ __attribute__((aligned(16))) uint8_t tiles[4 * kTileBytes];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t lr = lane & 15u, lg = lane >> 4;  // MFMA lane coordinates
-  const uint32_t h = blockIdx.y, kv = h / (d.heads / d.kv_heads);
-  // the last query blocks (the longest causal walks) first, so they do not start last
-  const uint32_t q0 = (gridDim.x - 1 - blockIdx.x) * kQ;
+  const uint32_t h = blockIdx.x, kv = h / (d.heads / d.kv_heads);
+  // the last query blocks (the longest causal walks) first, so they do not start last; heads vary
+  // fastest, which deals every length of walk to each XCD
+  const uint32_t q0 = (gridDim.y - 1 - blockIdx.y) * kQ;
   const uint32_t query = q0 + wave * 16 + lr;  // this lane's query (its column of S^T and O^T)
 
   // Q^T fragments (B operand of S^T = K Q^T): query lr, d 32 ks + 8 lg .. +8.
@@ -176,7 +148,7 @@ __global__ __launch_bounds__(256) void attention_kernel(const float* __restrict_
     }
   }
 
-  // O^T blocks (d 16 nd .. +16) in the D layout: lane holds d 16 nd + 4 lg + e of its query.
+  // O^T blocks (d 16 n .. +16) in the D layout: lane holds d 16 n + 4 lg + e of its query.
   f32x4 o[4];
 #pragma unroll
   for (int n = 0; n < 4; n++) o[n] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -194,47 +166,61 @@ __global__ __launch_bounds__(256) void attention_kernel(const float* __restrict_
   const uint32_t limit = d.query_begin + query;  // the last key this query sees
   // a tile wholly at or below the wave's first query's limit (and inside the keys) needs no mask
   const uint32_t open_end = min(d.query_begin + q0 + wave * 16 + 1, key_end);
-  // this lane's A-operand rows of S^T blocks n (even, odd): key 32 (n / 2) + 8 (lr / 4) + 4 (n % 2)
-  // + lr % 4, at its swizzled LDS row
-  const uint32_t krow = 8 * (lr >> 2) + (lr & 3u);
-  const uint32_t krows[2] = {ks_row(krow), ks_row(krow + 4)};
 
+  // The caches are read through buffer resources that end at the workgroup's last key: rows past it
+  // are zeros (a V row there must be finite - its weight is 0).
   const uint32_t pitch = d.kv_heads * kD * 2u;
-  const KVStream kst{egd::buffer(k_cache, key_end * pitch), egd::buffer(v_cache, key_end * pitch),
-                     (tid >> 2) * pitch + kv * kD * 2u + (tid & 3u) * 32u,
-                     (tid >> 4) * 4u * pitch + kv * kD * 2u + (tid & 15u) * 8u, pitch};
-  KVTile kvt;
-  if (ntiles) {
-    load_tile(kvt, kst, key_begin);
-    store_tile(kvt, Ks[0], Vt[0], tid);
-  }
-  __syncthreads();
+  const auto kr = egd::buffer(k_cache, key_end * pitch), vr = egd::buffer(v_cache, key_end * pitch);
+  const uint32_t trow = wave * 8 + (lane >> 3), slot = lane & 7u;  // this lane's row (and + 32) and LDS slot
+  const uint32_t koff = trow * pitch + kv * kD * 2u + 16u * (slot ^ ((trow >> 1) & 7u));
+  const uint32_t voff = trow * pitch + kv * kD * 2u + 16u * (slot ^ (trow & 6u));
+  auto load_tile = [&](uint32_t j0, uint32_t buf) {
+#pragma unroll
+    for (uint32_t i = 0; i < 2; i++) {
+      uint8_t* at = tiles + 2 * kTileBytes * buf + (4 * i + wave) * 1024u;
+      egd::load_to_lds(kr, at, (j0 + 32 * i) * pitch + koff);
+      egd::load_to_lds(vr, at + kTileBytes, (j0 + 32 * i) * pitch + voff);
+    }
+  };
+  auto settle = [&]() {
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt 0: the memory-to-LDS loads have landed
+    __syncthreads();
+  };
+  // LDS offsets of this lane's operand reads: K row lr, slots lg and lg + 4; V row 4 lg + lr / 4, d 4 (lr % 4).
+  const uint32_t ksw = (lr >> 1) & 7u, vrow = 4 * lg + (lr >> 2);
+  const uint32_t kat[2] = {lr * 128u + 16u * (lg ^ ksw), lr * 128u + 16u * ((lg + 4u) ^ ksw)};
+  uint32_t vat[4];
+#pragma unroll
+  for (uint32_t n = 0; n < 4; n++)
+    vat[n] = kTileBytes + vrow * 128u + 8u * (lr & 1u) + 16u * ((2 * n + ((lr >> 1) & 1u)) ^ (vrow & 6u));
+
+  if (ntiles) load_tile(key_begin, 0);
+  settle();
   for (uint32_t t = 0; t < ntiles; t++) {
     const uint32_t j0 = key_begin + t * kK, buf = t & 1u;
-    // the next tile's loads stay in flight through this tile's products
-    if (t + 1 < ntiles) load_tile(kvt, kst, j0 + kK);
+    const uint8_t* tile = tiles + 2 * kTileBytes * buf;
+    // (the other buffer was last read before the barrier that ended the previous tile)
+    if (t + 1 < ntiles) load_tile(j0 + kK, buf ^ 1u);
 
     f32x4 s[4];
 #pragma unroll
     for (int n = 0; n < 4; n++) {
       s[n] = f32x4{0.f, 0.f, 0.f, 0.f};
-      const uint32_t row = 32 * (n >> 1) + krows[n & 1];
 #pragma unroll
       for (int ks = 0; ks < 2; ks++) {
-        const half8 ka = *reinterpret_cast<const half8*>(&Ks[buf][row][32 * ks + 8 * lg]);
+        const half8 ka = *reinterpret_cast<const half8*>(tile + 2048u * n + kat[ks]);
         s[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qb[ks], s[n], 0, 0, 0);
       }
     }
 
     // Causal mask (tiles that cross a limit or the last key) and the online softmax: the lane's
-    // 16 scores, then the max over the 4 lanes holding the query (lanes lr, lr + 16, lr + 32,
-    // lr + 48).
+    // 16 scores, then the max over the 4 lanes holding the query.
     if (j0 + kK > open_end) {
 #pragma unroll
       for (int n = 0; n < 4; n++)
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-          const uint32_t j = j0 + 32 * (n >> 1) + 8 * lg + 4 * (n & 1) + e;
+          const uint32_t j = j0 + 16 * n + 4 * lg + e;
           if (!(j <= limit && j < key_end)) s[n][e] = kMasked;
         }
     }
@@ -243,21 +229,20 @@ __global__ __launch_bounds__(256) void attention_kernel(const float* __restrict_
     for (int n = 0; n < 4; n++)
 #pragma unroll
       for (int e = 0; e < 4; e++) mx = fmaxf(mx, s[n][e]);
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float mnew = fmaxf(m, mx);
+    const float mnew = fmaxf(m, max_of_query(mx));
     const float alpha = __builtin_amdgcn_exp2f((m - mnew) * kLog2e);
     // a query with no visible key yet (a split wholly past its causal limit) keeps nothing: its
     // exponent offset is pushed past f32's range below zero
     const float ml = mnew == kMasked ? 3.0e38f : mnew * kLog2e;
+    half8 pb[2];
     float sum = 0.f;
 #pragma unroll
     for (int n = 0; n < 4; n++)
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         const float p = __builtin_amdgcn_exp2f(fmaf(s[n][e], kLog2e, -ml));
-        s[n][e] = p;
         sum += p;
+        pb[n >> 1][4 * (n & 1) + e] = (_Float16)p;
       }
     l = l * alpha + sum;
     // the accumulators are rescaled only when some query of the wave found a larger max
@@ -269,19 +254,15 @@ __global__ __launch_bounds__(256) void attention_kernel(const float* __restrict_
 
     // O^T += V^T P^T over the two halves of the tile.
 #pragma unroll
-    for (int hh = 0; hh < 2; hh++) {
-      const half8 pb = half8{(_Float16)s[2 * hh][0],     (_Float16)s[2 * hh][1],     (_Float16)s[2 * hh][2],
-                             (_Float16)s[2 * hh][3],     (_Float16)s[2 * hh + 1][0], (_Float16)s[2 * hh + 1][1],
-                             (_Float16)s[2 * hh + 1][2], (_Float16)s[2 * hh + 1][3]};
+    for (int hh = 0; hh < 2; hh++)
 #pragma unroll
       for (int n = 0; n < 4; n++) {
-        const half8 va = *reinterpret_cast<const half8*>(&Vt[buf][16 * n + lr][32 * hh + 8 * lg]);
-        o[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pb, o[n], 0, 0, 0);
+        const uint8_t* at = tile + vat[n] + 4096u * hh;
+        const egd::s16x4 lo = egd::lds_read_transposed(at), hi = egd::lds_read_transposed(at + 2048u);
+        const half8 va = __builtin_bit_cast(half8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        o[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pb[hh], o[n], 0, 0, 0);
       }
-    }
-    // the other buffer was last read in the previous iteration, before the barrier that ended it
-    if (t + 1 < ntiles) store_tile(kvt, Ks[buf ^ 1u], Vt[buf ^ 1u], tid);
-    __syncthreads();
+    settle();
   }
 
   // the query's sum over its 4 lanes
@@ -323,23 +304,22 @@ __global__ __launch_bounds__(256) void attention_kernel(const float* __restrict_
 //   blocks, and a lane's o[0..3][e] are the four consecutive d = 16 g + 4 e .. +4.
 // K and V rows go from memory to LDS directly, the next tile's while this one is multiplied; K's 16-byte
 // slots are swizzled by the row. Sums stay short for their error's sake: a score is two chains of 32 products,
-// a tile's values are summed by themselves before they are added. MFMA-bound: 128 of 32 cycles per wave and tile. Against a workgroup per
-// query row with f32 FMAs: 256 queries at keys up to 2048, 14 / 2 heads, 208.7 -> 35.2 us on MI355X (RoPE,
-// append and combine included).
+// a tile's values are summed by themselves before they are added. MFMA-bound: 128 of 32 cycles per wave and
+// tile. Against a workgroup per query row with f32 FMAs: 256 queries at keys up to 2048, 14 / 2 heads,
+// 208.7 -> 35.3 us on MI355X (RoPE, append and combine included).
 constexpr uint32_t kF32Group = 8;  // query heads per kv head
 constexpr uint32_t kF32Tile = kK * kD * 4;  // bytes of a K (or V) tile
 
-__global__ __launch_bounds__(256) void attention_f32_kernel(const float* __restrict__ q_rope,
+__global__ __launch_bounds__(256, 2) void attention_f32_kernel(const float* __restrict__ q_rope,
                                                             const float* __restrict__ k_cache,
                                                             const float* __restrict__ v_cache, float* __restrict__ out,
                                                             eg_attention_prefill_dims d, Splits sp) {
-  __shared__ __attribute__((aligned(16))) uint8_t Ks[2][kF32Tile];
-  __shared__ __attribute__((aligned(16))) uint8_t Vs[2][kF32Tile];
+  __shared__ __attribute__((aligned(16))) uint8_t tiles[4 * kF32Tile];  // [buffer][K or V][key][d]
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t lr = lane & 15u, lg = lane >> 4;
-  const uint32_t h = blockIdx.y, kv = h / (d.heads / d.kv_heads);
-  const uint32_t q0 = (gridDim.x - 1 - blockIdx.x) * kQ;  // the longest causal walks first
+  const uint32_t h = blockIdx.x, kv = h / (d.heads / d.kv_heads);
+  const uint32_t q0 = (gridDim.y - 1 - blockIdx.y) * kQ;  // the longest causal walks first
   const uint32_t query = q0 + wave * 16 + lr;
 
   float qb[16];
@@ -380,8 +360,9 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(const float* __restr
     for (uint32_t i = 0; i < 4; i++) {
       const uint32_t r = (4 * i + wave) * 4 + lg, row = min(r, key_end - j0 - 1);
       const uint32_t at = (row * d.kv_heads + kv) * (kD * 4u);
-      egd::load_to_lds(kr, Ks[buf] + (4 * i + wave) * 1024u, at + 16u * (lr ^ (r & 15u)));
-      egd::load_to_lds(vr, Vs[buf] + (4 * i + wave) * 1024u, at + 16u * lr);
+      uint8_t* to = tiles + 2 * kF32Tile * buf + (4 * i + wave) * 1024u;
+      egd::load_to_lds(kr, to, at + 16u * (lr ^ (r & 15u)));
+      egd::load_to_lds(vr, to + kF32Tile, at + 16u * lr);
     }
   };
   auto settle = [&]() {
@@ -392,6 +373,7 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(const float* __restr
   settle();
   for (uint32_t t = 0; t < ntiles; t++) {
     const uint32_t j0 = key_begin + t * kK, buf = t & 1u;
+    const uint8_t *Ks = tiles + 2 * kF32Tile * buf, *Vs = Ks + kF32Tile;
     // (the other buffer was last read before the barrier that ended the previous tile)
     if (t + 1 < ntiles) load_tile(j0 + kK, buf ^ 1u);
 
@@ -403,7 +385,7 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(const float* __restr
       f32x4 ka[4];
 #pragma unroll
       for (uint32_t n = 0; n < 4; n++)
-        ka[n] = *reinterpret_cast<const f32x4*>(Ks[buf] + (16 * n + lr) * (kD * 4u) + 16u * ((4 * lg + j) ^ lr));
+        ka[n] = *reinterpret_cast<const f32x4*>(Ks + (16 * n + lr) * (kD * 4u) + 16u * ((4 * lg + j) ^ lr));
 #pragma unroll
       for (int c = 0; c < 4; c++)
 #pragma unroll
@@ -458,7 +440,7 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(const float* __restr
       bool finite = true;
 #pragma unroll
       for (uint32_t n = 0; n < 16; n++) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(Vs[buf] + (4 * n + lg) * (kD * 4u) + 16u * lr);
+        const f32x4 v = *reinterpret_cast<const f32x4*>(Vs + (4 * n + lg) * (kD * 4u) + 16u * lr);
 #pragma unroll
         for (int c = 0; c < 4; c++) finite = finite && isfinite(v[c]);
       }
@@ -469,7 +451,7 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(const float* __restr
       for (int n = 0; n < 4; n++)
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-          const f32x4 va = *reinterpret_cast<const f32x4*>(Vs[buf] + (16 * n + 4 * lg + e) * (kD * 4u) + 16u * lr);
+          const f32x4 va = *reinterpret_cast<const f32x4*>(Vs + (16 * n + 4 * lg + e) * (kD * 4u) + 16u * lr);
 #pragma unroll
           for (int nd = 0; nd < 4; nd++) ot[nd] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[nd], s[n][e], ot[nd], 0, 0, 0);
         }
@@ -484,7 +466,7 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(const float* __restr
             if (j0 + key > limit || j0 + key >= key_end) continue;
 #pragma unroll
             for (uint32_t c = 0; c < 4; c++) {
-              const f32x4 v = *reinterpret_cast<const f32x4*>(Vs[buf] + key * (kD * 4u) + 16u * (4 * lg + c));
+              const f32x4 v = *reinterpret_cast<const f32x4*>(Vs + key * (kD * 4u) + 16u * (4 * lg + c));
 #pragma unroll
               for (int nd = 0; nd < 4; nd++) ot[nd][c] = fmaf(p, v[nd], ot[nd][c]);
             }
@@ -652,11 +634,10 @@ int eg::attention_prefill_run(eg_context* ctx, const float* q_rope, const uint16
   if ((reinterpret_cast<uintptr_t>(q_rope) | reinterpret_cast<uintptr_t>(out)) & 15u)
     return eg::fail(ctx, EG_ERR_INVALID, "%s: q_rope and out must be 16-byte aligned", op);
   if (d.queries == 0) return EG_OK;
-  const uint32_t blocks = (d.queries + kQ - 1) / kQ;
   const uint64_t rows = (uint64_t)d.queries * d.heads;
   const Splits sp = splits_for(ctx, d);
-  hipLaunchKernelGGL(attention_kernel, dim3(blocks, d.heads, sp.count), dim3(256), 0, ctx->stream, q_rope, k_cache,
-                     v_cache, out, d, sp, out_bf16 ? 1u : 0u);
+  hipLaunchKernelGGL(attention_kernel, dim3(d.heads, (d.queries + kQ - 1) / kQ, sp.count), dim3(256), 0, ctx->stream,
+                     q_rope, k_cache, v_cache, out, d, sp, out_bf16 ? 1u : 0u);
   if (sp.o) {
     const uint64_t total = rows * kD;
     const uint32_t cblocks = (uint32_t)std::min<uint64_t>((total / 4 + 255) / 256, (uint64_t)ctx->cu_count * 8);
@@ -707,7 +688,7 @@ extern "C" int eg_attention_prefill_f32(eg_context* ctx, const float* q, const f
   const uint32_t blocks = (d.queries + kQ - 1) / kQ;
   const uint64_t rows = (uint64_t)d.queries * d.heads;
   const Splits sp = splits_for(ctx, d, 2);
-  hipLaunchKernelGGL(attention_f32_kernel, dim3(blocks, d.heads, sp.count), dim3(256), 0, ctx->stream, q_rope, k_cache,
+  hipLaunchKernelGGL(attention_f32_kernel, dim3(d.heads, blocks, sp.count), dim3(256), 0, ctx->stream, q_rope, k_cache,
                      v_cache, out, d, sp);
   if (sp.o) {
     const uint32_t cblocks = (uint32_t)std::min<uint64_t>((rows * kD / 4 + 255) / 256, (uint64_t)ctx->cu_count * 8);

@@ -1,4 +1,4 @@
-"""The f32 cache's chunk attention at the edges of its tiles (64 queries, 64 keys, key splits), and
+"""The chunk attention at the edges of its tiles (64 queries, 64 keys, key splits), over both cache types, and
 values that must not reach the queries that do not see them."""
 
 import numpy as np
@@ -18,15 +18,21 @@ def inputs(n, heads, kv_heads, seed):
 
 
 # one query at the first, the last and a tile's first key; 64 and 65 queries; chunks whose keys split
-# (5, 7 and 8 splits, some empty for some rows), one head per kv head
+# (5, 7 and 8 splits, some empty for some rows), one head per kv head. The f16 bar is the one of the
+# f16 kernel's own test: q and the softmax weights are rounded to f16 (2^-11 each).
+@pytest.mark.parametrize("cache", ["f32", "f16"])
 @pytest.mark.parametrize("begin,n,heads,kv_heads", [(0, 1, 14, 2), (64, 1, 14, 2), (2047, 1, 14, 2), (0, 65, 2, 2),
                                                      (63, 64, 3, 3), (1792, 256, 14, 2), (1000, 17, 8, 1), (0, 600, 4, 4)])
-def test_tile_edges(device, begin, n, heads, kv_heads):
+def test_tile_edges(device, begin, n, heads, kv_heads, cache):
     q, k, v, kc, vc = inputs(n, heads, kv_heads, 31 + begin + n)
-    got = run(device, q, k, v, kc.copy(), vc.copy(), begin, heads=heads, kv_heads=kv_heads)[1]
-    want = prefill_attention(q, k, v, kc, vc, begin, heads, kv_heads, D, THETA, cache="f32")[1]
+    if cache == "f16":
+        kc, vc = (c.astype(np.float16).astype(np.float32) for c in (kc, vc))
+    given = [c.copy() if cache == "f32" else c.astype(np.float16).view(np.uint16) for c in (kc, vc)]
+    got = run(device, q, k, v, *given, begin, heads=heads, kv_heads=kv_heads)[1]
+    want = prefill_attention(q, k, v, kc, vc, begin, heads, kv_heads, D, THETA, cache=cache)[1]
     rms = float(np.sqrt(np.mean(want.astype(np.float64) ** 2)))
-    assert_close(got.ravel(), want.ravel(), 1e-5 * rms, 2e-5, label=f"begin {begin} n {n} heads {heads}/{kv_heads}")
+    bar = (1e-5 * rms, 2e-5) if cache == "f32" else (1e-2 * rms, 1e-2)
+    assert_close(got.ravel(), want.ravel(), *bar, label=f"{cache} begin {begin} n {n} heads {heads}/{kv_heads}")
 
 
 @pytest.mark.parametrize("begin,n,bad", [(0, 100, 70), (1800, 100, 33)])
