@@ -116,7 +116,7 @@ __device__ __forceinline__ float max_of_query(float x) {
 // MI355X, 14 heads, this kernel alone: 2048 queries 38.8 -> 24.3 us, 256 at 1792 13.0 -> 10.8.
 constexpr uint32_t kTileBytes = kK * kD * 2;
 
-// (5 waves per SIMD, what LDS holds; the bound also keeps the accumulators out of the AGPRs.)
+// (5 waves per SIMD, what LDS holds.)
 __global__ __launch_bounds__(256, 5) void attention_kernel(const float* __restrict__ q_rope,
                                                            const uint16_t* __restrict__ k_cache,
                                                            const uint16_t* __restrict__ v_cache,
