@@ -47,38 +47,58 @@ __device__ __forceinline__ CT to_cache(float x) {
   else return float_to_half(x);
 }
 
+// One workgroup per row. Bound by a chain of latencies: the row's read, the double-precision angles and
+// the stores; so the pairs a thread takes first (all of a row of up to 16 heads of q and k) are read, and
+// v is moved, before the angles are computed: the operator on 256 queries at 1792, 14 + 2 heads, went
+// from 17.24 to 16.81 us over an f16 cache and from 35.41 to 34.97 over an f32 one.
 template <class CT>
 __global__ __launch_bounds__(256) void rope_append_kernel(const float* __restrict__ q, const float* __restrict__ k,
                                                           const float* __restrict__ v, float* __restrict__ q_rope,
                                                           CT* __restrict__ k_cache, CT* __restrict__ v_cache,
                                                           eg_attention_prefill_dims d) {
+  constexpr uint32_t kThreads = 256, kAhead = 2;
   const uint32_t i = blockIdx.x;  // query row of the chunk
   const uint32_t pos = d.query_begin + i;
   const uint32_t tid = threadIdx.x;
+  const uint32_t qn = d.heads * (kD / 2), kn = d.kv_heads * (kD / 2), vn = d.kv_heads * kD;
+  const float* qr = q + (size_t)i * d.heads * kD;
+  const float* kr = k + (size_t)i * d.kv_heads * kD;
+  const float* vr = v + (size_t)i * vn;
+  const auto pair_at = [&](uint32_t p) {
+    const uint32_t pp = p < qn ? p : p - qn;
+    const float* src = (p < qn ? qr : kr) + (size_t)(pp / (kD / 2)) * kD + pp % (kD / 2);
+    return make_float2(src[0], src[kD / 2]);
+  };
+  float2 ahead[kAhead];
+#pragma unroll
+  for (uint32_t j = 0; j < kAhead; j++) {
+    const uint32_t p = tid + j * kThreads;
+    ahead[j] = p < qn + kn ? pair_at(p) : make_float2(0.f, 0.f);
+  }
+  CT* vdst = v_cache + (size_t)pos * vn;
+  for (uint32_t p = tid; p < vn; p += kThreads) vdst[p] = to_cache<CT>(vr[p]);
   __shared__ double2 cs[kD / 2];
   if (tid < kD / 2) egd::rope_table<kD>(cs, tid, pos, d.theta);
   __syncthreads();
   const float scale = 1.0f / sqrtf((float)kD);  // a power of two: exact
-  const uint32_t qn = d.heads * (kD / 2), kn = d.kv_heads * (kD / 2);
-  for (uint32_t p = tid; p < qn + kn; p += blockDim.x) {
-    const bool is_q = p < qn;
-    const uint32_t pp = is_q ? p : p - qn;
+  const auto put = [&](uint32_t p, float2 x) {
+    const uint32_t pp = p < qn ? p : p - qn;
     const uint32_t head = pp / (kD / 2), e = pp % (kD / 2);
-    const float* src = is_q ? q + ((size_t)i * d.heads + head) * kD : k + ((size_t)i * d.kv_heads + head) * kD;
-    const float2 rr = egd::rotate(src[e], src[e + kD / 2], cs[e]);
-    const float ra = rr.x, rb = rr.y;
-    if (is_q) {
+    const float2 r = egd::rotate(x.x, x.y, cs[e]);
+    if (p < qn) {
       float* dst = q_rope + ((size_t)i * d.heads + head) * kD;
-      dst[e] = ra * scale;
-      dst[e + kD / 2] = rb * scale;
+      dst[e] = r.x * scale;
+      dst[e + kD / 2] = r.y * scale;
     } else {
       CT* dst = k_cache + ((size_t)pos * d.kv_heads + head) * kD;
-      dst[e] = to_cache<CT>(ra);
-      dst[e + kD / 2] = to_cache<CT>(rb);
+      dst[e] = to_cache<CT>(r.x);
+      dst[e + kD / 2] = to_cache<CT>(r.y);
     }
-  }
-  for (uint32_t p = tid; p < d.kv_heads * kD; p += blockDim.x)
-    v_cache[(size_t)pos * d.kv_heads * kD + p] = to_cache<CT>(v[(size_t)i * d.kv_heads * kD + p]);
+  };
+#pragma unroll
+  for (uint32_t j = 0; j < kAhead; j++)
+    if (tid + j * kThreads < qn + kn) put(tid + j * kThreads, ahead[j]);
+  for (uint32_t p = tid + kAhead * kThreads; p < qn + kn; p += kThreads) put(p, pair_at(p));
 }
 
 // Split partials: o [split][query][head][kD] (unnormalised), then m and l [split][query][head].
