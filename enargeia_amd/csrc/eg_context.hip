@@ -157,8 +157,6 @@ int eg_destroy(eg_context* ctx) {
   if (!ctx) return EG_OK;
   hipSetDevice(ctx->device);
   hipStreamSynchronize(ctx->own_stream);
-  if (ctx->rows_done) (void)hipEventDestroy(ctx->rows_done);
-  if (ctx->rows) (void)hipFree(ctx->rows);
   if (ctx->workspace) hipFree(ctx->workspace);
   hipStreamDestroy(ctx->own_stream);
   delete ctx;

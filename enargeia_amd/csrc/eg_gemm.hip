@@ -180,32 +180,16 @@ void to_bf16(eg_context* ctx, const float* x, size_t n, void* out) {
                      static_cast<uint4*>(out), n8);
 }
 
-// The context's buffer for bf16 rows, at least `bytes` long and free for work enqueued next on the
-// current stream: work on another stream that still reads it is waited for (on the device). NULL
-// where there is none: over its bound, during a capture (a graph would keep the address and replay
-// beside other work) or without memory; the caller then takes a tile that stages f32 rows.
-void* bf16_buffer(eg_context* ctx, uint64_t bytes) {
-  if (bytes > eg::kRowsBytes || ctx->capturing) return nullptr;
+// How many rows of k f32 values the workspace takes as bf16 at once, in whole tiles; 0: none, and the
+// launch stages f32 rows. The workspace's part for them is used on the context's own stream alone and
+// outside captures: every use is then ordered after the one before it, whatever other streams and
+// replayed graphs do beside it.
+uint32_t rows_at_once(const eg_context* ctx, uint32_t k, const Tile& t) {
+  if (ctx->stream != ctx->own_stream || ctx->capturing) return 0;
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(ctx->stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone) return nullptr;
-  if (ctx->rows_bytes < bytes) {
-    // growing: hipFree waits for the device
-    if (ctx->rows) (void)hipFree(ctx->rows);
-    ctx->rows = nullptr;
-    ctx->rows_bytes = 0;
-    const uint64_t size = std::min<uint64_t>(eg::kRowsBytes, (bytes + (8u << 20) - 1) / (8u << 20) * (8u << 20));
-    if (!ctx->rows_done && hipEventCreateWithFlags(&ctx->rows_done, hipEventDisableTiming) != hipSuccess) {
-      ctx->rows_done = nullptr;
-      return nullptr;
-    }
-    if (hipMalloc(&ctx->rows, size) != hipSuccess) {
-      ctx->rows = nullptr;
-      (void)hipGetLastError();
-      return nullptr;
-    }
-    ctx->rows_bytes = size;
-  }
-  return hipStreamWaitEvent(ctx->stream, ctx->rows_done, 0) == hipSuccess ? ctx->rows : nullptr;
+  if (hipStreamIsCapturing(ctx->stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone) return 0;
+  const uint64_t rows = eg::kRowsBytes / ((uint64_t)k * 2);
+  return (uint32_t)(rows / t.rows() * t.rows());
 }
 
 // ---- the choice of a tile -----------------------------------------------------------------------
@@ -260,32 +244,24 @@ uint64_t splits_for(const eg_context* ctx, const Tile& t, uint32_t m, uint64_t c
   return std::max<uint64_t>(1, std::min<uint64_t>(ctx->cu_count / tiles, chunks / t.kg));
 }
 
-// How a launch takes f32 rows of x (*x, m rows of k): the largest tiles take bf16 rows, rounded into
-// `scratch` (nullable; m k halves, 16-byte aligned) or the context's buffer; without either the tile
-// becomes 64 x 256, which stages f32 rows. Measured (MI355X): 2048 x 11008 x 4096 237 us with the rounding
+// Runs launch(tile, x, xm, first, rows) over f32 rows of x (m rows of k): one launch of all of them,
+// or - the largest tiles, which take bf16 rows - one per stretch of rows that the workspace holds as
+// bf16. Where it holds none, the tile of the same chunks and K groups that stages f32 rows takes
+// their place: slower, the same bits. Measured (MI355X): 2048 x 11008 x 4096 237 us with the rounding
 // launch, 361 with 64 x 256 on f32 rows.
-int stage_f32(eg_context* ctx, const void** x, uint32_t m, uint32_t k, void* scratch, Tile* t, bool* in_rows) {
-  *in_rows = false;
-  if (!t->bf16_only()) return kXF32;
-  void* rows = scratch;
-  if (!rows) {
-    rows = bf16_buffer(ctx, (uint64_t)m * k * 2);
-    *in_rows = rows != nullptr;
+template <class F>
+int over_f32_rows(eg_context* ctx, const Tile& t, const float* x, uint32_t m, uint32_t k, F launch) {
+  if (!t.bf16_only()) return launch(t, x, (int)kXF32, 0u, m);
+  const uint32_t at_once = rows_at_once(ctx, k, t);
+  if (!at_once) return launch(t.f32_form(), x, (int)kXF32, 0u, m);
+  void* const rows = ctx->workspace + eg::kRowsOffset;
+  for (uint32_t first = 0; first < m; first += at_once) {
+    const uint32_t n = std::min(at_once, m - first);
+    to_bf16(ctx, x + (size_t)first * k, (size_t)n * k, rows);
+    const int st = launch(t, rows, (int)kXBf16, first, n);
+    if (st != EG_OK) return st;
   }
-  if (!rows) {
-    *t = kTile64x256;
-    return kXF32;
-  }
-  to_bf16(ctx, static_cast<const float*>(*x), (size_t)m * k, rows);
-  *x = rows;
-  return kXBf16;
-}
-
-// After the launch that read the context's bf16 rows.
-int rows_used(eg_context* ctx, bool in_rows) {
-  if (!in_rows) return EG_OK;
-  const hipError_t err = hipEventRecord(ctx->rows_done, ctx->stream);
-  return err == hipSuccess ? EG_OK : eg::hip_fail(ctx, err, "matmul_q4_prefill");
+  return EG_OK;
 }
 
 // The workgroup grid of a tile over m rows and `cols` 64-column tiles, and the order its tiles are
@@ -373,26 +349,38 @@ int eg::prefill_gemm(eg_context* ctx, const float* x, const uint32_t* packed, co
   splits = (k + k_per_split - 1) / k_per_split;
   float* const partials = splits > 1 ? reinterpret_cast<float*>(eg::partials(ctx)) : nullptr;
   const float* const use_bias = dims->use_bias ? bias : nullptr;
+  // the splits' sum over `rows` rows from `first`
+  auto reduce = [&](uint32_t first, uint32_t rows) {
+    if (!partials) return;
+    const size_t at = (size_t)first * dims->out_stride;
+    const uint64_t total = (uint64_t)rows * n;
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>((total + 255) / 256, (uint64_t)ctx->cu_count * 8);
+    hipLaunchKernelGGL(prefill_reduce_kernel, dim3(blocks), dim3(256), 0, ctx->stream, partials, use_bias,
+                       residual ? residual + at : nullptr, out + at, rows, n, (uint32_t)splits, dims->out_stride,
+                       dims->out_offset);
+  };
   if (chunked) {
-    Args a{};
-    bool in_rows = false;
-    const void* rows = x;
-    const int xm = x_bf16 ? (int)kXBf16 : stage_f32(ctx, &rows, m, k, nullptr, &t, &in_rows);
-    a.x = rows;
-    a.partials = partials;
-    a.m = m;
-    a.k = k;
-    a.block_shift = (uint32_t)__builtin_ctz(bs);
-    a.blocks_per_row = dims->blocks_per_row;
-    a.k_per_split = k_per_split;
-    a.nmats = 1;
-    a.mats[0] = Mat{packed, scales, encoding == EG_ENC_SIGNED ? nullptr : zeros, use_bias, residual, out, n,
-                    dims->out_stride, dims->out_offset, tiles_n};
-    a.vec = partials ? n % 4 == 0 : vector_out(a.mats[0]);
-    set_grid(ctx, a, t, tiles_n, xm, bits);
-    const KernelFn fn = xm == kXBf16 ? pick_store_bf16(encoding, bits, t) : pick_store_f32(encoding, bits, t);
-    int st = launch_tile(ctx, op, fn, a, t, (uint32_t)splits);
-    if (st == EG_OK) st = rows_used(ctx, in_rows);
+    auto launch = [&](const Tile& tile, const void* rows_x, int xm, uint32_t first, uint32_t rows) {
+      const size_t at = (size_t)first * dims->out_stride;
+      Args a{};
+      a.x = rows_x;
+      a.partials = partials;
+      a.m = rows;
+      a.k = k;
+      a.block_shift = (uint32_t)__builtin_ctz(bs);
+      a.blocks_per_row = dims->blocks_per_row;
+      a.k_per_split = k_per_split;
+      a.nmats = 1;
+      a.mats[0] = Mat{packed, scales, encoding == EG_ENC_SIGNED ? nullptr : zeros, use_bias,
+                      residual ? residual + at : nullptr, out + at, n, dims->out_stride, dims->out_offset, tiles_n};
+      a.vec = partials ? n % 4 == 0 : vector_out(a.mats[0]);
+      set_grid(ctx, a, tile, tiles_n, xm, bits);
+      const KernelFn fn = xm == kXBf16 ? pick_store_bf16(encoding, bits, tile) : pick_store_f32(encoding, bits, tile);
+      const int st = launch_tile(ctx, op, fn, a, tile, (uint32_t)splits);
+      if (st == EG_OK) reduce(first, rows);
+      return st;
+    };
+    const int st = x_bf16 ? launch(t, x, (int)kXBf16, 0u, m) : over_f32_rows(ctx, t, x, m, k, launch);
     if (st != EG_OK) return st;
   } else {
     const ElementArgs a{x, packed, scales, encoding == EG_ENC_SIGNED ? nullptr : zeros, use_bias, residual, out, partials,
@@ -402,12 +390,7 @@ int eg::prefill_gemm(eg_context* ctx, const float* x, const uint32_t* packed, co
                                               : (kg == 4 ? element_kernel<EG_ENC_OFFSET_ZEROS, 4>
                                                          : element_kernel<EG_ENC_OFFSET_ZEROS, 1>);
     hipLaunchKernelGGL(fn, grid, block, 0, ctx->stream, a);
-  }
-  if (partials) {
-    const uint64_t total = (uint64_t)m * n;
-    const uint32_t blocks = (uint32_t)std::min<uint64_t>((total + 255) / 256, (uint64_t)ctx->cu_count * 8);
-    hipLaunchKernelGGL(prefill_reduce_kernel, dim3(blocks), dim3(256), 0, ctx->stream, partials, use_bias, residual, out,
-                       m, n, (uint32_t)splits, dims->out_stride, dims->out_offset);
+    reduce(0, m);
   }
   return eg::check_launch(ctx, op);
 }
@@ -447,11 +430,12 @@ bool fold_norm(const eg_context* ctx, uint32_t m, uint64_t cols, const float* no
   return norm && aligned16(norm) && cols * ((m + kTile - 1) / kTile) < (uint64_t)ctx->cu_count;
 }
 
-// The matrices (one_launch accepted them) as one launch; xm says how x is staged (kXNorm with
-// norm and eps: the rows' RMSNorm folded in).
-int launch_multi(eg_context* ctx, const void* x, uint32_t m, uint32_t k, uint32_t block_size, int encoding,
-                 const eg::PrefillMatrix* mats, uint32_t count, uint64_t cols, int xm, int epi, const Tile& t,
-                 const float* norm, float eps, const eg::PrefillRope* rope = nullptr, bool out_bf16 = false) {
+// The matrices (one_launch accepted them) as one launch over m rows of x, rows `first` on of the
+// outputs; xm says how x is staged (kXNorm with norm and eps: the rows' RMSNorm folded in).
+int launch_multi(eg_context* ctx, const void* x, uint32_t first, uint32_t m, uint32_t k, uint32_t block_size,
+                 int encoding, const eg::PrefillMatrix* mats, uint32_t count, uint64_t cols, int xm, int epi,
+                 const Tile& t, const float* norm, float eps, const eg::PrefillRope* rope = nullptr,
+                 bool out_bf16 = false) {
   Args a{};
   a.x = x;
   a.m = m;
@@ -465,10 +449,10 @@ int launch_multi(eg_context* ctx, const void* x, uint32_t m, uint32_t k, uint32_
   a.out_bf16 = out_bf16 ? 1u : 0u;
   if (rope) {
     a.rope = rope->table;
-    a.q_rope = rope->q_rope;
+    a.q_rope = rope->q_rope + (size_t)first * rope->q_heads * kCols;
     a.k_cache = rope->k_cache;
     a.v_cache = rope->v_cache;
-    a.rope_pos0 = rope->pos0;
+    a.rope_pos0 = rope->pos0 + first;
     a.q_heads = rope->q_heads;
     a.kv_heads = rope->kv_heads;
   }
@@ -476,9 +460,13 @@ int launch_multi(eg_context* ctx, const void* x, uint32_t m, uint32_t k, uint32_
   a.vec = 1;
   for (uint32_t i = 0; i < count; i++) {
     const eg::PrefillMatrix& w = mats[i];
+    // (out_bf16: `out` holds 2-byte values)
+    const size_t at = (size_t)first * w.out_stride;
     end = epi == kPair ? (uint32_t)cols : end + (w.n + kTile - 1) / kTile;
-    a.mats[i] = Mat{w.packed, w.scales, encoding == EG_ENC_SIGNED ? nullptr : w.zeros, w.bias, w.residual,
-                    w.out, w.n, w.out_stride, w.out_offset, end};
+    a.mats[i] = Mat{w.packed, w.scales, encoding == EG_ENC_SIGNED ? nullptr : w.zeros, w.bias,
+                    w.residual ? w.residual + at : nullptr,
+                    out_bf16 ? reinterpret_cast<float*>(reinterpret_cast<uint16_t*>(w.out) + at) : w.out + at, w.n,
+                    w.out_stride, w.out_offset, end};
     if (!vector_out(a.mats[i])) a.vec = 0;
   }
   set_grid(ctx, a, t, cols, xm, 4);
@@ -491,28 +479,21 @@ int launch_multi(eg_context* ctx, const void* x, uint32_t m, uint32_t k, uint32_
   return st != EG_OK ? st : eg::check_launch(ctx, "matmul_q4_prefill");
 }
 
-// x of a launch of tile *t: the rows' RMSNorm folded into it where that pays (kXNorm), else rmsnorm_rows
-// into `normed` - as bf16 rows where the context stages them - and f32 rows as stage_f32 takes them.
-// Sets *x, *xm and *in_rows.
-int prepare_x(eg_context* ctx, const void** x, uint32_t m, uint32_t k, uint64_t cols, Tile* t, const float* norm,
-              float eps, float* normed, void* scratch, int* xm, bool* in_rows) {
-  *in_rows = false;
-  if (fold_norm(ctx, m, cols, norm)) {
-    *xm = kXNorm;
-    return EG_OK;
-  }
+// Runs launch(tile, x, xm, first, rows) over the rows, RMS-normalised first where norm is given: folded
+// into the launch where that pays (kXNorm), else by rmsnorm_rows into `normed` - as bf16 rows where the
+// context stages them.
+template <class F>
+int over_rows(eg_context* ctx, const Tile& t, const float* x, uint32_t m, uint32_t k, uint64_t cols, const float* norm,
+              float eps, float* normed, F launch) {
+  if (fold_norm(ctx, m, cols, norm)) return launch(t, x, (int)kXNorm, 0u, m);
   if (norm) {
     if (!normed) return eg::fail(ctx, EG_ERR_INVALID, "matmul_q4_prefill: RMSNorm needs a buffer for the normed rows");
-    const int st = eg::rmsnorm_rows(ctx, static_cast<const float*>(*x), norm, m, k, eps, normed, ctx->prefill_xb16);
+    const int st = eg::rmsnorm_rows(ctx, x, norm, m, k, eps, normed, ctx->prefill_xb16);
     if (st != EG_OK) return st;
-    *x = normed;
-    if (ctx->prefill_xb16) {
-      *xm = kXBf16;
-      return EG_OK;
-    }
+    if (ctx->prefill_xb16) return launch(t, normed, (int)kXBf16, 0u, m);
+    x = normed;
   }
-  *xm = stage_f32(ctx, x, m, k, scratch, t, in_rows);
-  return EG_OK;
+  return over_f32_rows(ctx, t, x, m, k, launch);
 }
 
 }  // namespace
@@ -527,13 +508,11 @@ int eg::prefill_gemm_multi(eg_context* ctx, const float* x, uint32_t m, uint32_t
   // One launch where the chunked staging takes every matrix and no matrix would split K;
   // otherwise (and for anything the single path must reject with its own message) one each.
   if ((count >= 2 || norm) && one_launch(x, m, k, block_size, encoding, bits, mats, count, &cols, &tile_cols)) {
-    Tile t = tile_for(ctx, m, tile_cols, k, block_size);
-    int xm = kXF32;
-    bool in_rows = false;
-    const void* rows = x;
-    int st = prepare_x(ctx, &rows, m, k, cols, &t, norm, eps, normed, nullptr, &xm, &in_rows);
-    if (st == EG_OK) st = launch_multi(ctx, rows, m, k, block_size, encoding, mats, count, cols, xm, kStore, t, norm, eps);
-    return st == EG_OK ? rows_used(ctx, in_rows) : st;
+    return over_rows(ctx, tile_for(ctx, m, tile_cols, k, block_size), x, m, k, cols, norm, eps, normed,
+                     [&](const Tile& t, const void* rows_x, int xm, uint32_t first, uint32_t rows) {
+                       return launch_multi(ctx, rows_x, first, rows, k, block_size, encoding, mats, count, cols, xm,
+                                           kStore, t, norm, eps);
+                     });
   }
   if (norm) {
     if (!normed) return eg::fail(ctx, EG_ERR_INVALID, "%s: RMSNorm needs a buffer for the normed rows", op);
@@ -569,15 +548,12 @@ int eg::prefill_qkv_rope(eg_context* ctx, const float* x, uint32_t m, uint32_t k
       mats[1].n != rope.kv_heads * kTile || mats[2].n != rope.kv_heads * kTile ||
       !one_launch(x, m, k, block_size, encoding, bits, mats, 3, &cols, &tile_cols))
     return EG_OK;
-  Tile t = tile_for(ctx, m, tile_cols, k, block_size);
-  int xm = kXF32;
-  bool in_rows = false;
-  const void* rows = x;
-  int st = prepare_x(ctx, &rows, m, k, cols, &t, norm, eps, normed, nullptr, &xm, &in_rows);
-  if (st != EG_OK) return st;
   *done = true;
-  st = launch_multi(ctx, rows, m, k, block_size, encoding, mats, 3, cols, xm, kRope, t, norm, eps, &rope);
-  return st == EG_OK ? rows_used(ctx, in_rows) : st;
+  return over_rows(ctx, tile_for(ctx, m, tile_cols, k, block_size), x, m, k, cols, norm, eps, normed,
+                   [&](const Tile& t, const void* rows_x, int xm, uint32_t first, uint32_t rows) {
+                     return launch_multi(ctx, rows_x, first, rows, k, block_size, encoding, mats, 3, cols, xm, kRope, t,
+                                         norm, eps, &rope);
+                   });
 }
 
 int eg::prefill_gemm_swiglu(eg_context* ctx, const float* x, uint32_t m, uint32_t k, uint32_t block_size,
@@ -601,17 +577,12 @@ int eg::prefill_gemm_swiglu(eg_context* ctx, const float* x, uint32_t m, uint32_
     if (st == EG_OK && m > 0 && n > 0) st = eg::silu_mul_rows(ctx, scratch, m, n, out, out_bf16);
     return st;
   }
-  Tile t = tile_for(ctx, m, tile_cols, k, block_size);
-  int xm = kXF32;
-  bool in_rows = false;
-  const void* rows = x;
-  // the scratch rows ([m][2 n] floats) are free here: they hold the bf16 rows of x where those fit
-  void* const spare = (uint64_t)2 * n * 4 >= (uint64_t)k * 2 && aligned16(scratch) ? scratch : nullptr;
-  int st = prepare_x(ctx, &rows, m, k, (n + 31) / 32, &t, norm, eps, normed, spare, &xm, &in_rows);
-  if (st != EG_OK) return st;
-  st = launch_multi(ctx, rows, m, k, block_size, encoding, pair, 2, (n + 31) / 32, xm, kPair, t, norm, eps, nullptr,
-                    out_bf16);
-  return st == EG_OK ? rows_used(ctx, in_rows) : st;
+  const uint64_t pairs = (n + 31) / 32;
+  return over_rows(ctx, tile_for(ctx, m, tile_cols, k, block_size), x, m, k, pairs, norm, eps, normed,
+                   [&](const Tile& t, const void* rows_x, int xm, uint32_t first, uint32_t rows) {
+                     return launch_multi(ctx, rows_x, first, rows, k, block_size, encoding, pair, 2, pairs, xm, kPair, t,
+                                         norm, eps, nullptr, out_bf16);
+                   });
 }
 
 extern "C" int eg_matmul_q4_prefill_swiglu(eg_context* ctx, const float* x, const uint32_t* gate_packed,

@@ -45,11 +45,6 @@ struct eg_context {
   // The prefill GEMM's tile (BK, MF, WN, KG of its kernel, and the K splits) forced by
   // EG_PREFILL_TILE="bk,mf,wn,kg[,splits]" for tuning sweeps; zeros: chosen per launch.
   int gemm_tile[5] = {0, 0, 0, 0, 0};
-  // bf16 rows of a prefill GEMM's f32 x (eg_gemm.hip): grown on use up to eg::kRowsBytes, freed with
-  // the context; the event after its last use.
-  void* rows = nullptr;
-  size_t rows_bytes = 0;
-  hipEvent_t rows_done = nullptr;
   // chunk attention's key split: at most this many 64-key tiles per workgroup, and a small grid
   // split up to this many workgroups per CU
   // the SwiGLU pair as one launch of paired gate|up tiles (false: gate | up, then silu_mul_rows)
@@ -91,12 +86,13 @@ int hip_fail(eg_context* ctx, hipError_t err, const char* what);
 // Workspace layout (bytes from ctx->workspace). Fixed offsets; sizes bound the op limits.
 constexpr size_t kStateOffset = 256;           // small per-op state
 constexpr size_t kPartialsOffset = 8192;       // per-workgroup partials
-constexpr size_t kWorkspaceBytes = 64u << 20;  // 64 MiB
+constexpr size_t kRowsOffset = 64u << 20;      // bf16 rows of a prefill GEMM's f32 x (eg_gemm.hip)
+constexpr size_t kWorkspaceBytes = 128u << 20;
 
 inline uint8_t* state(eg_context* ctx) { return ctx->workspace + kStateOffset; }
 inline uint8_t* partials(eg_context* ctx) { return ctx->workspace + kPartialsOffset; }
-constexpr size_t kPartialsBytes = kWorkspaceBytes - kPartialsOffset;
-constexpr size_t kRowsBytes = 64u << 20;  // bound of eg_context::rows
+constexpr size_t kPartialsBytes = kRowsOffset - kPartialsOffset;
+constexpr size_t kRowsBytes = kWorkspaceBytes - kRowsOffset;
 
 // Second stage of every multi-workgroup argmax: one workgroup reduces `groups` partials
 // (value bits, index) in a fixed order into result = [index, value bits]. A separate launch

@@ -105,7 +105,7 @@ typedef struct eg_sample_dims {
 /* ---- context ---------------------------------------------------------------------------- */
 
 /* Replaces initGPU (src/gpu/device.ts:116): binds HIP device `device`, creates a stream at the
- * default priority and a small workspace for cross-workgroup reductions. */
+ * default priority and a 128 MiB workspace (cross-workgroup partials, bf16 rows of a prefill's x). */
 EG_API int eg_create(int device, eg_context** out_ctx);
 EG_API int eg_destroy(eg_context* ctx);
 /* Last error message of this context, or of the calling thread when ctx is NULL. */
@@ -158,8 +158,9 @@ EG_API int eg_matmul_q4_prefill(eg_context* ctx, const float* x, const uint32_t*
  *   out[r*n + j] = silu(x[r] . gate_j) * (x[r] . up_j),  silu(g) = g / (1 + e^-g),  j < n
  * with the prefill GEMM's arithmetic (bf16 operands, f32 accumulation). gate and up share the
  * dims (n rows of k each; use_bias must be 0, out_stride n, out_offset 0), the encoding and
- * the bits. One launch where the chunked staging takes both matrices and K is at most 1984;
- * otherwise gate | up side by side into scratch ([m][2n] floats, required) and silu_mul. */
+ * the bits. One launch where the chunked staging takes both matrices and K is at most 1984, which
+ * leaves scratch as it is; otherwise gate | up side by side into scratch ([m][2n] floats, required)
+ * and silu_mul. */
 EG_API int eg_matmul_q4_prefill_swiglu(eg_context* ctx, const float* x, const uint32_t* gate_packed,
                                        const float* gate_scales, const uint32_t* gate_zeros,
                                        const uint32_t* up_packed, const float* up_scales,
