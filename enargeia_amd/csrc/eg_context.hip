@@ -123,8 +123,10 @@ int eg_create(int device, eg_context** out_ctx) {
     }
   }
   if (const char* g = std::getenv("EG_PREFILL_TILE")) {
-    int* t = ctx->gemm_tile;
-    if (std::sscanf(g, "%d,%d,%d,%d,%d", &t[0], &t[1], &t[2], &t[3], &t[4]) < 4) std::memset(t, 0, sizeof(ctx->gemm_tile));
+    int t[5] = {0, 0, 0, 0, 0};
+    if (std::sscanf(g, "%d,%d,%d,%d,%d", &t[0], &t[1], &t[2], &t[3], &t[4]) >= 4 && t[4] >= 0 && t[4] <= 64 &&
+        eg::prefill_tile_known(t))
+      std::memcpy(ctx->gemm_tile, t, sizeof(t));
   }
   err = hipMalloc(&ctx->workspace, eg::kWorkspaceBytes);
   if (err != hipSuccess) {

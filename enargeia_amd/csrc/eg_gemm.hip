@@ -219,7 +219,9 @@ uint64_t tile_count(const Tile& t, uint32_t m, uint64_t cols) {
 // and 128 x 128 comes before 64 x 256, whose weights are dequantized for half the rows. Blocks of 16
 // codes need the 64-deep chunks.
 Tile tile_for(const eg_context* ctx, uint32_t m, uint64_t cols, uint32_t k, uint32_t bs) {
-  if (ctx->gemm_tile[0]) return Tile{ctx->gemm_tile[0], ctx->gemm_tile[1], ctx->gemm_tile[2], ctx->gemm_tile[3]};
+  // (a lane's BK / 2 codes take two scales)
+  if (ctx->gemm_tile[0] && bs * 4 >= (uint32_t)ctx->gemm_tile[0])
+    return Tile{ctx->gemm_tile[0], ctx->gemm_tile[1], ctx->gemm_tile[2], ctx->gemm_tile[3]};
   const uint64_t cus = (uint64_t)ctx->cu_count;
   const bool deep = k >= 2048;
   auto fits = [&](const Tile& t) { return tile_count(t, m, cols) <= cus; };
@@ -289,6 +291,12 @@ bool vector_out(const Mat& w) {
 }
 
 }  // namespace
+
+bool eg::prefill_tile_known(const int* tile) {
+  for (const Tile& t : kTiles)
+    if (t.bk == tile[0] && t.mf == tile[1] && t.wn == tile[2] && t.kg == tile[3]) return true;
+  return false;
+}
 
 bool eg::prefill_chunked(uint32_t m, uint32_t n, uint32_t k, uint32_t bs, int bits, const void* x,
                          const uint32_t* packed) {
@@ -424,10 +432,11 @@ bool one_launch(const float* x, uint32_t m, uint32_t k, uint32_t block_size, int
 
 // Whether a launch folds the rows' RMSNorm in: only under one 64 x 64 tile per CU (latency-bound),
 // where the extra staging work (the weight multiply and the squares) is hidden; a launch that fills
-// the device is bound by that work, and a separate rmsnorm_rows launch costs less. (These launches
-// take tiles of up to 64 x 128.)
-bool fold_norm(const eg_context* ctx, uint32_t m, uint64_t cols, const float* norm) {
-  return norm && aligned16(norm) && cols * ((m + kTile - 1) / kTile) < (uint64_t)ctx->cu_count;
+// the device is bound by that work, and a separate rmsnorm_rows launch costs less. (The tiles of these
+// launches, 64 x 64 at most, have the kernel; a forced one may not.)
+bool fold_norm(const eg_context* ctx, const Tile& t, uint32_t m, uint64_t cols, const float* norm) {
+  return norm && aligned16(norm) && cols * ((m + kTile - 1) / kTile) < (uint64_t)ctx->cu_count && t.wn <= 2 &&
+         !t.bf16_only();
 }
 
 // The matrices (one_launch accepted them) as one launch over m rows of x, rows `first` on of the
@@ -485,7 +494,7 @@ int launch_multi(eg_context* ctx, const void* x, uint32_t first, uint32_t m, uin
 template <class F>
 int over_rows(eg_context* ctx, const Tile& t, const float* x, uint32_t m, uint32_t k, uint64_t cols, const float* norm,
               float eps, float* normed, F launch) {
-  if (fold_norm(ctx, m, cols, norm)) return launch(t, x, (int)kXNorm, 0u, m);
+  if (fold_norm(ctx, t, m, cols, norm)) return launch(t, x, (int)kXNorm, 0u, m);
   if (norm) {
     if (!normed) return eg::fail(ctx, EG_ERR_INVALID, "matmul_q4_prefill: RMSNorm needs a buffer for the normed rows");
     const int st = eg::rmsnorm_rows(ctx, x, norm, m, k, eps, normed, ctx->prefill_xb16);

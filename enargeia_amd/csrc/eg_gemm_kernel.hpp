@@ -575,6 +575,8 @@ struct Tile {
 // The tiles: {BK, MF, WN, KG}. eg_gemm.hip's tile_for chooses among them.
 constexpr Tile kTile32x64{128, 1, 1, 4}, kTile64x64{128, 2, 1, 4}, kTile64x128{64, 2, 2, 2}, kTile64x128Deep{128, 2, 2, 4},
     kTile64x256{128, 2, 4, 1}, kTile128x128{128, 4, 2, 2}, kTile128x256{128, 4, 4, 1}, kTile32x64Fine{64, 1, 1, 4};
+constexpr Tile kTiles[] = {kTile32x64,  kTile64x64,   kTile64x128,  kTile64x128Deep,
+                           kTile64x256, kTile128x128, kTile128x256, kTile32x64Fine};
 
 // The largest take bf16 rows of x only (f32 rows staged through registers do not fit beside the sums;
 // f32_form then takes them), and the RMSNorm is folded into launches of few tiles only, which take the small ones.

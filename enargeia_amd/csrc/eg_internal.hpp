@@ -43,7 +43,8 @@ struct eg_context {
   uint32_t stamp_capacity = 0;
   uint32_t stamp_next = 0;
   // The prefill GEMM's tile (BK, MF, WN, KG of its kernel, and the K splits) forced by
-  // EG_PREFILL_TILE="bk,mf,wn,kg[,splits]" for tuning sweeps; zeros: chosen per launch.
+  // EG_PREFILL_TILE="bk,mf,wn,kg[,splits]" for tuning sweeps and tests, for the launches that have that
+  // kernel; zeros (and anything but one of its tiles): chosen per launch.
   int gemm_tile[5] = {0, 0, 0, 0, 0};
   // chunk attention's key split: at most this many 64-key tiles per workgroup, and a small grid
   // split up to this many workgroups per CU
@@ -261,6 +262,8 @@ int attention_prefill_run(eg_context* ctx, const float* q_rope, const uint16_t* 
 // launches that can stage bf16 rows of x).
 bool prefill_chunked(uint32_t m, uint32_t n, uint32_t k, uint32_t block_size, int bits, const void* x,
                      const uint32_t* packed);
+// Whether bk, mf, wn, kg name one of the prefill GEMM's tiles.
+bool prefill_tile_known(const int* tile);
 int check_attention_prefill(eg_context* ctx, const char* op, const eg_attention_prefill_dims* dims);
 // The SwiGLU pair: out[r][j] = SiLU(x[r] . gate_j + bias) * (x[r] . up_j + bias), j < gate.n, rows
 // gate.n apart (the outputs and strides in gate and up are ignored). One launch of paired tiles
