@@ -128,10 +128,16 @@ int eg_create(int device, eg_context** out_ctx) {
         eg::prefill_tile_known(t))
       std::memcpy(ctx->gemm_tile, t, sizeof(t));
   }
-  err = hipMalloc(&ctx->workspace, eg::kWorkspaceBytes);
-  if (err != hipSuccess) {
+  auto undo = [&]() {
+    if (ctx->rows) (void)hipFree(ctx->rows);
+    if (ctx->workspace) (void)hipFree(ctx->workspace);
     hipStreamDestroy(ctx->own_stream);
     delete ctx;
+  };
+  err = hipMalloc(&ctx->workspace, eg::kWorkspaceBytes);
+  if (err == hipSuccess) err = hipMalloc(&ctx->rows, eg::kRowsBytes);
+  if (err != hipSuccess) {
+    undo();
     return hip_fail(nullptr, err, "eg_create: workspace");
   }
   ctx->workspace_bytes = eg::kWorkspaceBytes;
@@ -139,16 +145,12 @@ int eg_create(int device, eg_context** out_ctx) {
   err = hipMemset(ctx->workspace, 0, eg::kPartialsOffset);
   if (err == hipSuccess) err = hipDeviceSynchronize();
   if (err != hipSuccess) {
-    hipFree(ctx->workspace);
-    hipStreamDestroy(ctx->own_stream);
-    delete ctx;
+    undo();
     return hip_fail(nullptr, err, "eg_create: workspace init");
   }
   if (eg::noalloc_scratch_init(ctx) != EG_OK) {
     fail(nullptr, EG_ERR_DEVICE, "%s", ctx->error);
-    hipFree(ctx->workspace);
-    hipStreamDestroy(ctx->own_stream);
-    delete ctx;
+    undo();
     return EG_ERR_DEVICE;
   }
   *out_ctx = ctx;
@@ -159,7 +161,8 @@ int eg_destroy(eg_context* ctx) {
   if (!ctx) return EG_OK;
   hipSetDevice(ctx->device);
   hipStreamSynchronize(ctx->own_stream);
-  if (ctx->workspace) hipFree(ctx->workspace);
+  if (ctx->rows) (void)hipFree(ctx->rows);
+  if (ctx->workspace) (void)hipFree(ctx->workspace);
   hipStreamDestroy(ctx->own_stream);
   delete ctx;
   return EG_OK;

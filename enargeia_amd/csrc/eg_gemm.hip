@@ -180,9 +180,8 @@ void to_bf16(eg_context* ctx, const float* x, size_t n, void* out) {
                      static_cast<uint4*>(out), n8);
 }
 
-// How many rows of k f32 values the workspace takes as bf16 at once, in whole tiles; 0: none, and the
-// launch stages f32 rows. The workspace's part for them is used on the context's own stream alone and
-// outside captures: every use is then ordered after the one before it, whatever other streams and
+// How many rows of k f32 values the context's buffer takes as bf16 at once, in whole tiles; 0: none, and
+// the launch stages f32 rows. The buffer is used on the context's own stream alone and outside captures: every use is then ordered after the one before it, whatever other streams and
 // replayed graphs do beside it.
 uint32_t rows_at_once(const eg_context* ctx, uint32_t k, const Tile& t) {
   if (ctx->stream != ctx->own_stream || ctx->capturing) return 0;
@@ -247,8 +246,8 @@ uint64_t splits_for(const eg_context* ctx, const Tile& t, uint32_t m, uint64_t c
 }
 
 // Runs launch(tile, x, xm, first, rows) over f32 rows of x (m rows of k): one launch of all of them,
-// or - the largest tiles, which take bf16 rows - one per stretch of rows that the workspace holds as
-// bf16. Where it holds none, the tile of the same chunks and K groups that stages f32 rows takes
+// or - the largest tiles, which take bf16 rows - one per stretch of rows that the context's buffer
+// holds. Where it holds none, the tile of the same chunks and K groups that stages f32 rows takes
 // their place: slower, the same bits. Measured (MI355X): 2048 x 11008 x 4096 237 us with the rounding
 // launch, 361 with 64 x 256 on f32 rows.
 template <class F>
@@ -256,7 +255,7 @@ int over_f32_rows(eg_context* ctx, const Tile& t, const float* x, uint32_t m, ui
   if (!t.bf16_only()) return launch(t, x, (int)kXF32, 0u, m);
   const uint32_t at_once = rows_at_once(ctx, k, t);
   if (!at_once) return launch(t.f32_form(), x, (int)kXF32, 0u, m);
-  void* const rows = ctx->workspace + eg::kRowsOffset;
+  void* const rows = ctx->rows;
   for (uint32_t first = 0; first < m; first += at_once) {
     const uint32_t n = std::min(at_once, m - first);
     to_bf16(ctx, x + (size_t)first * k, (size_t)n * k, rows);

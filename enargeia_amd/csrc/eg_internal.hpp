@@ -22,6 +22,10 @@ struct eg_context {
   // element is written before it is read within one op, so it needs no clearing.
   uint8_t* workspace = nullptr;
   size_t workspace_bytes = 0;
+  // bf16 rows of a prefill GEMM's f32 x (eg_gemm.hip), eg::kRowsBytes. Not the workspace's other half: in
+  // one allocation of 128 MiB the chunk attention's splits took longer to write and merge (1 query at
+  // 3227, 16 splits: 17.3 us for 16.5).
+  void* rows = nullptr;
   bool capturing = false;
   // This device's copy of the fixed scratch array of eg_lm_head_argmax_noalloc (resolved by
   // eg::noalloc_scratch_init at creation; shared by every context on the device).
@@ -87,13 +91,12 @@ int hip_fail(eg_context* ctx, hipError_t err, const char* what);
 // Workspace layout (bytes from ctx->workspace). Fixed offsets; sizes bound the op limits.
 constexpr size_t kStateOffset = 256;           // small per-op state
 constexpr size_t kPartialsOffset = 8192;       // per-workgroup partials
-constexpr size_t kRowsOffset = 64u << 20;      // bf16 rows of a prefill GEMM's f32 x (eg_gemm.hip)
-constexpr size_t kWorkspaceBytes = 128u << 20;
+constexpr size_t kWorkspaceBytes = 64u << 20;  // 64 MiB
 
 inline uint8_t* state(eg_context* ctx) { return ctx->workspace + kStateOffset; }
 inline uint8_t* partials(eg_context* ctx) { return ctx->workspace + kPartialsOffset; }
-constexpr size_t kPartialsBytes = kRowsOffset - kPartialsOffset;
-constexpr size_t kRowsBytes = kWorkspaceBytes - kRowsOffset;
+constexpr size_t kPartialsBytes = kWorkspaceBytes - kPartialsOffset;
+constexpr size_t kRowsBytes = 64u << 20;  // eg_context::rows
 
 // Second stage of every multi-workgroup argmax: one workgroup reduces `groups` partials
 // (value bits, index) in a fixed order into result = [index, value bits]. A separate launch

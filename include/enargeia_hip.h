@@ -105,7 +105,7 @@ typedef struct eg_sample_dims {
 /* ---- context ---------------------------------------------------------------------------- */
 
 /* Replaces initGPU (src/gpu/device.ts:116): binds HIP device `device`, creates a stream at the
- * default priority and a 128 MiB workspace (cross-workgroup partials, bf16 rows of a prefill's x). */
+ * default priority and its workspaces (64 MiB of cross-workgroup partials, 64 of a prefill's rows). */
 EG_API int eg_create(int device, eg_context** out_ctx);
 EG_API int eg_destroy(eg_context* ctx);
 /* Last error message of this context, or of the calling thread when ctx is NULL. */

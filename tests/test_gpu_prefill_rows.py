@@ -1,4 +1,4 @@
-"""The prefill GEMM's bf16 rows of f32 x: where the tile wants them they are held in the workspace
+"""The prefill GEMM's bf16 rows of f32 x: where the tile wants them they are held in the buffer
 that the context was created with, a stretch of rows at a time, and calls that may not use it - under a
 capture, on a caller's stream - stage the f32 rows themselves with the same sums, to the bit."""
 
@@ -111,7 +111,7 @@ def test_a_callers_stream_gives_the_same_bits(tile, m, n, k, bits):
         owner.close()
 
 
-def test_rows_past_the_workspace():
+def test_rows_past_the_buffer():
     """4500 rows of 8192 are 70 MiB as bf16: two stretches, the same bits as two calls."""
     m, n, k, half = 4500, 200, 8192, 2250
     dev = device_with("128,4,2,2,1")
