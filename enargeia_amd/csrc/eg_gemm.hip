@@ -284,9 +284,9 @@ int launch_tile(eg_context* ctx, const char* op, KernelFn fn, const Args& a, con
   return EG_OK;
 }
 
-// Whether a matrix's outputs (and residual) take 16-byte accesses.
+// Whether a matrix's outputs take 16-byte stores.
 bool vector_out(const Mat& w) {
-  return w.n % 4 == 0 && w.out_stride % 4 == 0 && w.out_offset % 4 == 0 && aligned16(w.out) && aligned16(w.residual);
+  return w.n % 4 == 0 && w.out_stride % 4 == 0 && w.out_offset % 4 == 0 && aligned16(w.out);
 }
 
 }  // namespace
@@ -380,7 +380,6 @@ int eg::prefill_gemm(eg_context* ctx, const float* x, const uint32_t* packed, co
       a.nmats = 1;
       a.mats[0] = Mat{packed, scales, encoding == EG_ENC_SIGNED ? nullptr : zeros, use_bias,
                       residual ? residual + at : nullptr, out + at, n, dims->out_stride, dims->out_offset, tiles_n};
-      a.vec = partials ? n % 4 == 0 : vector_out(a.mats[0]);
       set_grid(ctx, a, tile, tiles_n, xm, bits);
       const KernelFn fn = xm == kXBf16 ? pick_store_bf16(encoding, bits, tile) : pick_store_f32(encoding, bits, tile);
       const int st = launch_tile(ctx, op, fn, a, tile, (uint32_t)splits);

@@ -32,6 +32,7 @@ namespace eg_gemm {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // 16 bytes at any float's address
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 
@@ -58,7 +59,7 @@ struct Args {
   uint32_t tiles_x, tiles_y;  // workgroup tiles
   uint32_t nmats;             // matrices in mats (> 1: no K split)
   uint32_t xcd;               // order in which tiles are dealt to the XCDs (see tile_of)
-  uint32_t vec;               // outputs (and residuals) take 16-byte accesses, n a multiple of 4
+  uint32_t vec;               // kPair: out takes 16-byte (out_bf16: 8-byte) stores, n a multiple of 4
   const float* norm;          // kXNorm: x is RMS-normalised per row with these weights (no K split)
   float eps;
   // kRope launches (q | k | v, 64-column tiles = heads): q rows rotated and scaled by 1/8 into
@@ -400,7 +401,8 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_kernel(Args a) {
     const uint32_t buf = it & 1u;
     Weights wb;
     multiply(group + KG * it, buf, wa, wb);
-    store_x(buf ^ 1u);
+    // (not the last: it would wait for loads past K to convert their zeros; 1 x 64 x 256 4.4 -> 3.8 us)
+    if (it + 1 < iters) store_x(buf ^ 1u);
     settle();
     wa = wb;
   }
@@ -428,15 +430,38 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_kernel(Args a) {
 #pragma unroll
     for (int e = 0; e < 4; e++) c.cs[EPI == kRope ? e : 0] = a.rope[(size_t)(a.rope_pos0 + row) * 32u + 8u * p + 4u * g + e];
   };
+  // 1 / rms of row r of the tile, the groups' sums of squares added in group order
+  auto inv_rms = [&](uint32_t r) {
+    float sum = row_ss[0][r];
+#pragma unroll
+    for (int q = 1; q < (XM == kXNorm ? KG : 1); q++) sum += row_ss[q][r];
+    return 1.0f / sqrtf(sum / (float)a.k + a.eps);
+  };
+  // One value of a row, and columns col .. +4 of it in one access wherever the rows start.
+  auto store1 = [&](uint32_t row, uint32_t col, float v) {
+    if (a.partials) {
+      a.partials[((size_t)blockIdx.y * a.m + row) * w0.n + col] = v;
+      return;
+    }
+    const size_t o = (size_t)row * w0.out_stride + col + w0.out_offset;
+    w0.out[o] = v + (w0.bias ? w0.bias[col] : 0.f) + (w0.residual ? w0.residual[o] : 0.f);
+  };
+  auto store4 = [&](uint32_t row, uint32_t col, f32x4 v) {
+    if (a.partials) {
+      *reinterpret_cast<f32x4u*>(a.partials + ((size_t)blockIdx.y * a.m + row) * w0.n + col) = v;
+      return;
+    }
+    const size_t o = (size_t)row * w0.out_stride + col + w0.out_offset;
+    const f32x4 res = w0.residual ? (f32x4)*reinterpret_cast<const f32x4u*>(w0.residual + o) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = v[e] + (w0.bias ? w0.bias[col + e] : 0.f) + res[e];
+    *reinterpret_cast<f32x4u*>(w0.out + o) = v;
+  };
   auto finish = [&](uint32_t i, uint32_t p, f32x4 lo, f32x4 hi, const Angles& an) {
     const uint32_t r = 32u * i + lr, row = m0 + r;
     if (!active || row >= a.m) return;
     if (XM == kXNorm) {
-      // 1 / rms of the row, the groups' sums of squares added in group order
-      float sum = row_ss[0][r];
-#pragma unroll
-      for (int q = 1; q < (XM == kXNorm ? KG : 1); q++) sum += row_ss[q][r];
-      const float inv = 1.0f / sqrtf(sum / (float)a.k + a.eps);
+      const float inv = inv_rms(r);
       lo *= inv;
       hi *= inv;
     }
@@ -494,30 +519,13 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_kernel(Args a) {
 #pragma unroll
     for (int h = 0; h < 2; h++) {
       const uint32_t col = n0 + 8u * p + 32u * h + 4u * g;
-      f32x4 v = h ? hi : lo;
-      if (a.partials) {
-        float* dst = a.partials + ((size_t)blockIdx.y * a.m + row) * w0.n + col;
-        if (a.vec) {
-          if (col < w0.n) *reinterpret_cast<f32x4*>(dst) = v;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; e++)
-            if (col + e < w0.n) dst[e] = v[e];
-        }
-        continue;
-      }
-      const size_t o = (size_t)row * w0.out_stride + col + w0.out_offset;
-      if (a.vec) {
-        if (col >= w0.n) continue;
-        f32x4 res = w0.residual ? *reinterpret_cast<const f32x4*>(w0.residual + o) : f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int e = 0; e < 4; e++) v[e] = v[e] + (w0.bias ? w0.bias[col + e] : 0.f) + res[e];
-        *reinterpret_cast<f32x4*>(w0.out + o) = v;
+      const f32x4 v = h ? hi : lo;
+      if (col + 4 <= w0.n) {
+        store4(row, col, v);
       } else {
 #pragma unroll
         for (int e = 0; e < 4; e++)
-          if (col + e < w0.n)
-            w0.out[o + e] = v[e] + (w0.bias ? w0.bias[col + e] : 0.f) + (w0.residual ? w0.residual[o + e] : 0.f);
+          if (col + e < w0.n) store1(row, col + e, v[e]);
       }
     }
   };
@@ -533,6 +541,46 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_kernel(Args a) {
         finish(i, p, run(acc[0][i], p), run(acc[1][i], p), an);
         __builtin_amdgcn_sched_barrier(0);  // one unit at a time: together they spill
       }
+  } else if constexpr (EPI == kStore) {
+    // Every wave's sums into LDS (the last barrier ended the staging), then rows of 64 columns shared out
+    // over the groups: 16 lanes take the 16 runs of four columns of a row, 256 bytes in one store. Run
+    // (f, p, g) of row lr is kept at slot lane ^ (4 f + p + 8 g) of its 64, which puts the 16 on different
+    // banks. The run that n cuts comes after them, a value per lane: with its stores in every unrolled step
+    // the launch took 1.2 to 2.5 us longer (749 x 1086 x 320 8.8 us, 749 x 1088 7.7), for instruction fetches.
+    f32x4* const sums = reinterpret_cast<f32x4*>(lds);
+    auto at = [&](uint32_t q, uint32_t f, uint32_t u, uint32_t l) {
+      return ((q * WN + wn) * (8u * MF) + f * (4 * MF) + u) * 64u + (l ^ (4u * f + (u & 3u) + 8u * (l >> 5)));
+    };
+#pragma unroll
+    for (int f = 0; f < 2; f++)
+#pragma unroll
+      for (int u = 0; u < 4 * MF; u++) sums[at(group, f, u, lane)] = run(acc[f][u / 4], u % 4);
+    __syncthreads();
+    if (!active) return;
+    const uint32_t c = lane & 15u, f = c >> 3, p = (c >> 1) & 3u;
+#pragma unroll
+    for (uint32_t v = 0; v < 8u * MF / KG; v++) {
+      const uint32_t r = (group + v * KG) * 4u + (lane >> 4), u = (r >> 5) * 4u + p, l = (r & 31u) + 32u * (c & 1u);
+      f32x4 x = sums[at(0, f, u, l)];
+#pragma unroll
+      for (int q = 1; q < KG; q++) x += sums[at(q, f, u, l)];
+      if (m0 + r >= a.m || n0 + 4u * c + 4u > w0.n) continue;
+      if (XM == kXNorm) x *= inv_rms(r);
+      store4(m0 + r, n0 + 4u * c, x);
+    }
+    const uint32_t cut = w0.n & ~3u;  // the cut run's first column
+    if (n0 + kCols <= cut || cut == w0.n) return;
+    const uint32_t cc = cut - n0, r = (group * 64u + lane) % TM;
+    if (m0 + r >= a.m) return;
+    const uint32_t cf = cc >> 5, cu = (r >> 5) * 4u + ((cc >> 3) & 3u), cl = (r & 31u) + 32u * ((cc >> 2) & 1u);
+#pragma unroll 1
+    for (uint32_t e = (group * 64u + lane) / TM; e < (w0.n & 3u); e += KG * 64u / TM) {
+      float x = sums[at(0, cf, cu, cl)][e];
+#pragma unroll
+      for (int q = 1; q < KG; q++) x += sums[at(q, cf, cu, cl)][e];
+      if (XM == kXNorm) x *= inv_rms(r);
+      store1(m0 + r, cut + e, x);
+    }
   } else {
     // every wave's sums into LDS as its lanes hold them (the last barrier ended the staging), then
     // the units shared out over the groups

@@ -10,6 +10,7 @@ import oracle
 from conftest import assert_close
 from enargeia_amd import kernels as K
 from test_gpu_prefill import model_tol, run_prefill
+from test_gpu_prefill_rows import device_with
 
 pytestmark = pytest.mark.gpu
 
@@ -37,6 +38,30 @@ def test_tile_edges_match_the_bf16_model(device, m, n, k, bits, fmt, bs):
     got = run_prefill(device, x, q, bias, m)
     model = oracle.linear_q_bf16_fast(x, q, bias, m)
     assert_close(got, model, *model_tol(model), label=f"{m}x{n}x{k} int{bits} {fmt} {bs}")
+
+
+TILES = {"32 x 64 fine": "64,1,1,4", "32 x 64": "128,1,1,4", "64 x 64": "128,2,1,4", "64 x 128": "64,2,2,2",
+         "64 x 128 deep": "128,2,2,4", "64 x 256": "128,2,4,1", "128 x 128": "128,4,2,2", "128 x 256": "128,4,4,1"}
+
+
+@pytest.mark.parametrize("tile", list(TILES))
+@pytest.mark.parametrize("n", [65, 126, 191, 320])
+def test_cut_runs_of_columns(tile, n):
+    """n that leaves one, two or three columns of a run of four, or none: every column is stored, and
+    nothing past the rows; 70 and 150 rows, the last chunk of K short."""
+    k = 416
+    dev = device_with(TILES[tile])
+    try:
+        for m, fmt, bits in ((70, "sym", 4), (150, "ref", 8)):
+            x = oracle.normal_floats(m * k, m, 1.0)
+            q = weights(n, k, bits, fmt, 32)
+            bias = oracle.normal_floats(n, 3, 0.02)
+            got = run_prefill(dev, x, q, bias, m, out_len=m * n + 300)
+            model = oracle.linear_q_bf16_fast(x, q, bias, m)
+            assert_close(got[:m * n], model, *model_tol(model), label=f"{tile} n {n} m {m}")
+            assert not got[m * n:].any()
+    finally:
+        dev.close()
 
 
 @pytest.mark.parametrize("m,n,k", [(70, 96, 96), (450, 4600, 96), (1030, 4170, 96)])
