@@ -199,41 +199,84 @@ uint64_t tile_count(const Tile& t, uint32_t m, uint64_t cols) {
   return ((cols + t.wn - 1) / t.wn) * ((m + t.rows() - 1) / t.rows());
 }
 
-// The tile of a launch over m rows, `cols` 64-column tiles and k: the smallest that still covers the
-// matrix in one workgroup per CU (a second round of these workgroups costs more than larger tiles),
-// and the largest where none does. Large tiles spread the dequantization over more rows; small ones
-// fill the device and, with four groups of waves on alternate chunks of K, shorten the serial chain.
-// Measured on MI355X with bf16 rows of x (us; int4 sym at K = 896, ref format else):
-//                        32x64  64x64  64x128  64x256  128x128  128x256
-//     512 x  896 x  896    7.6    8.6    11.4       -        -        -   (224, 112, 56 tiles)
-//    1024 x  896 x  896    9.4    9.0    11.7    15.3        -        -   (448, 224, 112, 64)
-//     128 x 9728 x  896   12.5   15.4    11.9    15.3        -        -   (608, 304, 152, 76)
-//     256 x 9728 x  896   18.7   22.1    16.8    16.1     17.5     23.0   (1216, 608, 304, 152, 152, 76)
-//     512 x 9728 x  896      -      -    25.7    24.6     32.5     24.6   (-, -, 608, 304, 304, 152)
-//    2048 x  896 x 4864   63.2   61.0    41.6    45.5     44.2     41.9   (deep 64x128: 224 tiles)
-//    1024 x 4096 x 4096      -      -    75.3    75.6     54.5     59.4   (-, -, 512, 256, 256, 128)
-//    2048 x 4096 x 11008     -      -       -   305.8    233.1    213.5   (-, -, -, 512, 512, 256)
-// K from 2048 (16 chunks) is long: 64 x 128 then takes eight waves and deeper chunks (41.6 against 54.4 us
-// at 2048 x 896 x 4864; at K = 896 the four-wave form, 12.6 against 13.9 us for f32 rows at 256 x 4864),
-// and 128 x 128 comes before 64 x 256, whose weights are dequantized for half the rows. Blocks of 16
-// codes need the 64-deep chunks.
-Tile tile_for(const eg_context* ctx, uint32_t m, uint64_t cols, uint32_t k, uint32_t bs) {
-  // (a lane's BK / 2 codes take two scales)
-  if (ctx->gemm_tile[0] && bs * 4 >= (uint32_t)ctx->gemm_tile[0])
-    return Tile{ctx->gemm_tile[0], ctx->gemm_tile[1], ctx->gemm_tile[2], ctx->gemm_tile[3]};
+// The tile of a launch over m rows and k. A sum's order is that of the chunks and K groups (BK, KG), so
+// those are chosen for `cols` 64-column tiles - of one matrix, where a launch holds several of one shape:
+// gate and up as a pair, in one launch and on their own give the same bits - and the rows and columns
+// for the `launch_cols` tiles that the launch has.
+//
+// Up to K = 2048 the smallest tile that still covers the matrix in one workgroup per CU (a second round
+// of these workgroups costs more than larger tiles), and the largest where none does: large tiles spread
+// the dequantization over more rows, small ones fill the device and, with four groups of waves on alternate
+// chunks of K, shorten the serial chain. The small ones take 64-deep chunks ("fine") up to K = 768 and where
+// those leave fewer idle steps to the groups (K of 1025 to 1280), and at 769 to 896, where both leave
+// the same, from half a workgroup per CU on (a gate|up pair is then twice that, and its launches fold the
+// norm: 64 x 4864 x 896 as a pair 10.4 us fine, 11.3 else). Measured on MI355X (us; f32 rows, int4 sym;
+// workgroups of 32x64 | 64x64 | 64x128 | 64x256):
+//                     32x64 fine  32x64  64x64 fine  64x64  64x128  64x256  128x256
+//     64 x 1024 x  320       5.1    5.3         6.7    7.3     7.9    10.6     13.5   (32)
+//    128 x 4864 x  640       8.3    9.6         8.1    9.3     9.8    13.4     20.8   (304 | 152)
+//    512 x  896 x  896       7.1    7.0         8.9    9.3    11.2    16.0     24.2   (224 | 112)
+//    128 x 4864 x  896       9.7    9.9         9.1    9.4    11.3    16.1     23.9   (304 | 152)
+//    128 x 4864 x 1152      10.8   12.2        10.1   11.2    12.8    18.5     27.1   (304 | 152)
+//    384 x 1536 x 1536      15.4   13.4        11.8   11.2    16.5    22.2     35.9   (288 | 144)
+//    256 x 4864 x  896      13.0   14.3        13.5   17.6    11.7    16.4     24.2   (608 | 304 | 152)
+//    256 x 9728 x  896      19.1   21.8        19.3   25.8    17.1    17.1     25.0   (1216 | 608 | 304 | 152)
+//   2048 x 1152 x  896, q|k|v (RoPE)
+//                           23.2   25.0        23.7   27.4    23.8    22.1     29.5   (1152 | 576 | 288 | 160)
+//    200 x 8960 x 1536      26.5   24.6        27.3   31.1    28.0    23.2     35.8   (980 | 560 | 280 | 140)
+//    512 x 9728 x  896         -      -        29.5   42.7    25.7    26.1     27.8   (2432 | 1216 | 608 | 304)
+//   2048 x 9728 x  896, gate|up (bf16 rows): 64x256 64, 128x256 58
+//
+// From K = 2048 on the grid may be split over K, at 2.3 us and the partial sums' traffic: 32 x 64 where
+// three splits of it fill the CUs, or where it needs none and K is short enough; else larger tiles with more
+// splits, which dequantize each weight for more rows (with no more than 32 rows none has more). Measured
+// (splits in brackets; f32 rows, bf16 ones for 896 x 4864):
+//                       32x64     64x64     64x128 long  64x128 deep  128x128   128x256
+//    100 x 2048 x 2048  9.0 (2)   11.1 (4)  11.7 (4)     14.7 (4)     14.2 (8)  16.5 (8)
+//    256 x 2048 x 2048  10.1      12.8      15.0 (4)     18.2 (2)     21.2 (4)  24.5 (6)
+//     64 x 4096 x 4096  13.9 (2)  14.1 (4)  15.2 (4)     18.0 (4)     19.8 (8)  22.4 (8)
+//     16 x 4096 x 11008 16.3 (4)  20.0 (4)  19.2 (8)     20.6 (8)     24.1 (8)  31.9 (8)
+//    256 x  896 x 4864  14.9 (2)  13.8 (4)  16.6 (8)     16.5 (6)     19.8 (8)  22.8 (8)
+//    100 x 1536 x 8960  22.1 (2)  20.2 (4)  18.8 (8)     22.1 (6)     25.3 (8)  33.0 (8)
+//     64 x 4096 x 11008 26.3 (2)  23.9 (4)  22.2 (8)     23.8 (8)     26.7 (8)  35.0 (8)
+//   1024 x  896 x 4864  31.2      24.6      26.5 (4)     25.8 (2)     25.5 (4)  30.3 (8)
+//   2048 x  896 x 4864  60.1      48.7      41.8 (2)     35.7         36.6 (2)  39.8 (4)
+//   1024 x 4096 x 4096  109       89.7      61.5         64.4         48.1      56.5 (2)
+//   2048 x 4096 x 11008 -         420       276          300          221       207
+//
+// RoPE's epilogue (angles, rotation, f16 rows) grows with a tile's rows: 32 up to two workgroups per CU
+// (q|k|v of 600 rows, fine: 11.6 us; 64 x 64, not fine: 13.5). Blocks of 16 codes need the 64-deep chunks.
+Tile tile_for(const eg_context* ctx, uint32_t m, uint64_t cols, uint32_t k, uint32_t bs, uint64_t launch_cols,
+              int epi) {
+  if (ctx->gemm_tile[0]) {
+    // (a lane's BK / 2 codes take two scales)
+    const Tile t{ctx->gemm_tile[0], ctx->gemm_tile[1], ctx->gemm_tile[2], ctx->gemm_tile[3]};
+    if (bs * 4 >= (uint32_t)t.bk && (epi == kStore || !t.store_only())) return t;
+  }
   const uint64_t cus = (uint64_t)ctx->cu_count;
-  const bool deep = k >= 2048;
-  auto fits = [&](const Tile& t) { return tile_count(t, m, cols) <= cus; };
-  if (bs < 32) return fits(kTile32x64Fine) ? kTile32x64Fine : kTile64x128;
-  // two workgroups of 32 x 64 (or of 64 x 128) fit on a CU: they may outnumber the CUs a little; over a
-  // long K 32 x 64 only pays where the grid is split anyway
-  if (tile_count(kTile32x64, m, cols) <= (deep ? cus / 2 : cus * 5 / 4)) return kTile32x64;
+  auto count = [&](const Tile& t) { return tile_count(t, m, cols); };
+  auto fits = [&](const Tile& t) { return count(t) <= cus; };
+  // of two tiles of 32 and 64 rows: 32 where that is a workgroup per CU, 64 where that is one or the
+  // workgroups are many in any case (two of the others fit on a CU)
+  auto rows = [&](const Tile& low, const Tile& high) {
+    const uint64_t n = tile_count(low, m, launch_cols);
+    if (n <= cus || (epi == kRope && n <= 2 * cus)) return low;
+    return tile_count(high, m, launch_cols) <= cus || n > 3 * cus ? high : low;
+  };
+  const uint64_t n = count(kTile32x64);
+  if (bs < 32) return fits(kTile64x64Fine) ? rows(kTile32x64Fine, kTile64x64Fine) : kTile64x128;
+  if (k < 2048) {
+    const bool fine = k <= 768 || (k <= 896 && n > cus / 2) || (k > 1024 && k <= 1280);
+    if (fits(kTile64x64) || (m <= 32 && n <= 2 * cus))
+      return fine ? rows(kTile32x64Fine, kTile64x64Fine) : rows(kTile32x64, kTile64x64);
+    if (fits(kTile64x128)) return kTile64x128;
+    return fits(kTile64x256) ? kTile64x256 : kTile128x256;
+  }
+  if (n <= cus / 3 || (n <= cus && (m <= 32 || k <= (n <= cus / 2 ? 3584u : 4096u)))) return kTile32x64;
+  if (n <= cus / 2 && k >= 8192) return kTile64x128Long;
   if (fits(kTile64x64)) return kTile64x64;
-  if (deep ? fits(kTile64x128Deep) : tile_count(kTile64x128, m, cols) <= cus * 5 / 4)
-    return deep ? kTile64x128Deep : kTile64x128;
-  if (deep && fits(kTile128x128)) return kTile128x128;
-  if (!deep && fits(kTile64x256)) return kTile64x256;
-  return kTile128x256;
+  if (fits(kTile64x128Deep)) return kTile64x128Deep;
+  return fits(kTile128x128) ? kTile128x128 : kTile128x256;
 }
 
 // Ranges K is split into over the grid: where the tiles leave CUs idle over a long K, down to one
@@ -341,7 +384,7 @@ int eg::prefill_gemm(eg_context* ctx, const float* x, const uint32_t* packed, co
   uint32_t step = kBK;
   int kg = 1;
   if (chunked) {
-    t = tile_for(ctx, m, tiles_n, k, bs);
+    t = tile_for(ctx, m, tiles_n, k, bs, tiles_n, kStore);
     splits = splits_for(ctx, t, m, tiles_n, k);
     step = t.bk;
   } else {
@@ -406,8 +449,7 @@ namespace {
 // Whether matrices sharing x run in ONE launch: the chunked staging takes every one of them and
 // no K split is wanted (K under 2048). Sets the total of their 64-column tiles, and the number the
 // launch's tile is chosen for: matrices of one shape take the tile that one of them alone takes, so
-// that gate and up as a pair, in one launch and on their own give the same bits (4% slower at 256
-// rows of the pair than its own best tile, equal from 512); others their total.
+// that gate and up as a pair, in one launch and on their own give the same bits; others their total.
 bool one_launch(const float* x, uint32_t m, uint32_t k, uint32_t block_size, int encoding, int bits,
                 const eg::PrefillMatrix* mats, uint32_t count, uint64_t* tiles_n, uint64_t* tile_cols) {
   bool ok = count >= 1 && count <= kMaxSegs && m > 0 && x && bits == 4 &&
@@ -433,8 +475,7 @@ bool one_launch(const float* x, uint32_t m, uint32_t k, uint32_t block_size, int
 // the device is bound by that work, and a separate rmsnorm_rows launch costs less. (The tiles of these
 // launches, 64 x 64 at most, have the kernel; a forced one may not.)
 bool fold_norm(const eg_context* ctx, const Tile& t, uint32_t m, uint64_t cols, const float* norm) {
-  return norm && aligned16(norm) && cols * ((m + kTile - 1) / kTile) < (uint64_t)ctx->cu_count && t.wn <= 2 &&
-         !t.bf16_only();
+  return norm && aligned16(norm) && cols * ((m + kTile - 1) / kTile) < (uint64_t)ctx->cu_count && t.folds_norm();
 }
 
 // The matrices (one_launch accepted them) as one launch over m rows of x, rows `first` on of the
@@ -515,7 +556,7 @@ int eg::prefill_gemm_multi(eg_context* ctx, const float* x, uint32_t m, uint32_t
   // One launch where the chunked staging takes every matrix and no matrix would split K;
   // otherwise (and for anything the single path must reject with its own message) one each.
   if ((count >= 2 || norm) && one_launch(x, m, k, block_size, encoding, bits, mats, count, &cols, &tile_cols)) {
-    return over_rows(ctx, tile_for(ctx, m, tile_cols, k, block_size), x, m, k, cols, norm, eps, normed,
+    return over_rows(ctx, tile_for(ctx, m, tile_cols, k, block_size, cols, kStore), x, m, k, cols, norm, eps, normed,
                      [&](const Tile& t, const void* rows_x, int xm, uint32_t first, uint32_t rows) {
                        return launch_multi(ctx, rows_x, first, rows, k, block_size, encoding, mats, count, cols, xm,
                                            kStore, t, norm, eps);
@@ -556,7 +597,7 @@ int eg::prefill_qkv_rope(eg_context* ctx, const float* x, uint32_t m, uint32_t k
       !one_launch(x, m, k, block_size, encoding, bits, mats, 3, &cols, &tile_cols))
     return EG_OK;
   *done = true;
-  return over_rows(ctx, tile_for(ctx, m, tile_cols, k, block_size), x, m, k, cols, norm, eps, normed,
+  return over_rows(ctx, tile_for(ctx, m, tile_cols, k, block_size, cols, kRope), x, m, k, cols, norm, eps, normed,
                    [&](const Tile& t, const void* rows_x, int xm, uint32_t first, uint32_t rows) {
                      return launch_multi(ctx, rows_x, first, rows, k, block_size, encoding, mats, 3, cols, xm, kRope, t,
                                          norm, eps, &rope);
@@ -585,7 +626,7 @@ int eg::prefill_gemm_swiglu(eg_context* ctx, const float* x, uint32_t m, uint32_
     return st;
   }
   const uint64_t pairs = (n + 31) / 32;
-  return over_rows(ctx, tile_for(ctx, m, tile_cols, k, block_size), x, m, k, pairs, norm, eps, normed,
+  return over_rows(ctx, tile_for(ctx, m, tile_cols, k, block_size, pairs, kPair), x, m, k, pairs, norm, eps, normed,
                    [&](const Tile& t, const void* rows_x, int xm, uint32_t first, uint32_t rows) {
                      return launch_multi(ctx, rows_x, first, rows, k, block_size, encoding, pair, 2, pairs, xm, kPair, t,
                                          norm, eps, nullptr, out_bf16);

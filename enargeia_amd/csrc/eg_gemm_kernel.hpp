@@ -615,19 +615,23 @@ using KernelFn = void (*)(Args);
 struct Tile {
   int bk, mf, wn, kg;
   uint32_t rows() const { return 32u * mf; }
+  // which kernels there are: the largest take bf16 rows of x only (f32 rows staged through registers do
+  // not fit beside the sums), those for a long K store plain results, and the RMSNorm is folded into
+  // launches of few tiles only, which take the small ones
   bool bf16_only() const { return mf * wn * kg >= 16; }
+  bool store_only() const { return bk == 128 && wn == 2; }
+  bool folds_norm() const { return wn == 1 || (wn == 2 && bk == 64); }
   // the tile that takes a bf16_only one's f32 rows: its chunks and K groups, half its rows or columns
   Tile f32_form() const { return kg == 4 ? Tile{bk, mf, wn / 2, kg} : Tile{bk, mf / 2, wn, kg}; }
 };
 
 // The tiles: {BK, MF, WN, KG}. eg_gemm.hip's tile_for chooses among them.
-constexpr Tile kTile32x64{128, 1, 1, 4}, kTile64x64{128, 2, 1, 4}, kTile64x128{64, 2, 2, 2}, kTile64x128Deep{128, 2, 2, 4},
-    kTile64x256{128, 2, 4, 1}, kTile128x128{128, 4, 2, 2}, kTile128x256{128, 4, 4, 1}, kTile32x64Fine{64, 1, 1, 4};
-constexpr Tile kTiles[] = {kTile32x64,  kTile64x64,   kTile64x128,  kTile64x128Deep,
-                           kTile64x256, kTile128x128, kTile128x256, kTile32x64Fine};
+constexpr Tile kTile32x64{128, 1, 1, 4}, kTile64x64{128, 2, 1, 4}, kTile64x128{64, 2, 2, 2}, kTile64x128Long{128, 2, 2, 2},
+    kTile64x128Deep{128, 2, 2, 4}, kTile64x256{128, 2, 4, 1}, kTile128x128{128, 4, 2, 2}, kTile128x256{128, 4, 4, 1},
+    kTile32x64Fine{64, 1, 1, 4}, kTile64x64Fine{64, 2, 1, 4};
+constexpr Tile kTiles[] = {kTile32x64,  kTile64x64,   kTile64x128,  kTile64x128Long, kTile64x128Deep,
+                           kTile64x256, kTile128x128, kTile128x256, kTile32x64Fine,  kTile64x64Fine};
 
-// The largest take bf16 rows of x only (f32 rows staged through registers do not fit beside the sums;
-// f32_form then takes them), and the RMSNorm is folded into launches of few tiles only, which take the small ones.
 template <int ENC, int BITS, int XM, int EPI>
 KernelFn pick_tile(const Tile& t) {
 #define EG_GEMM_CASE(B, M, W, G) \
@@ -636,15 +640,18 @@ KernelFn pick_tile(const Tile& t) {
   EG_GEMM_CASE(128, 2, 1, 4)
   EG_GEMM_CASE(64, 2, 2, 2)
   EG_GEMM_CASE(64, 1, 1, 4)
+  EG_GEMM_CASE(64, 2, 1, 4)
   if constexpr (XM != kXNorm) {
     EG_GEMM_CASE(128, 2, 4, 1)
-  }
-  if constexpr (XM == kXF32) {
-    EG_GEMM_CASE(128, 2, 2, 2)  // (f32_form of 128 x 128)
+    if constexpr (EPI == kStore) {
+      EG_GEMM_CASE(128, 2, 2, 2)
+    }
   }
   if constexpr (XM == kXBf16) {
-    EG_GEMM_CASE(128, 2, 2, 4)
-    EG_GEMM_CASE(128, 4, 2, 2)
+    if constexpr (EPI == kStore) {
+      EG_GEMM_CASE(128, 2, 2, 4)
+      EG_GEMM_CASE(128, 4, 2, 2)
+    }
     EG_GEMM_CASE(128, 4, 4, 1)
   }
 #undef EG_GEMM_CASE

@@ -14,7 +14,8 @@ from test_gpu_prefill_rows import device_with
 
 pytestmark = pytest.mark.gpu
 
-TILES = ["128,1,1,4", "128,2,1,4", "64,2,2,2", "128,2,2,4", "128,2,4,1", "128,4,2,2", "128,4,4,1", "64,1,1,4"]
+TILES = ["128,1,1,4", "128,2,1,4", "64,2,2,2", "128,2,2,2", "128,2,2,4", "128,2,4,1", "128,4,2,2", "128,4,4,1", "64,1,1,4",
+         "64,2,1,4"]
 
 
 @pytest.mark.parametrize("value", ["", "64", "128,2,0,1", "128,2,4,0", "0,0,0,0", "128,3,1,4", "32,1,1,4", "128,1,1,4,-2",

@@ -1,7 +1,8 @@
-"""The prefill GEMM's tiles at their edges: one shape per tile the library chooses (32 x 64, 64 x 64,
-64 x 128 shallow and deep, 64 x 256, 128 x 128, 128 x 256, and the 64-deep chunks of 16-code blocks),
-with rows and columns that do not fill the last tile, K that does not fill the last chunk, both
-encodings and both code widths, against the oracle's bf16 model at the f32 sums' 1e-4."""
+"""The prefill GEMM's tiles at their edges: rows and columns that do not fill the last tile, K that does
+not fill the last chunk, both encodings and both code widths, against the oracle's bf16 model at the
+f32 sums' 1e-4 - at shapes for which the library chooses each tile, and with each tile forced."""
+
+import os
 
 import numpy as np
 import pytest
@@ -9,7 +10,7 @@ import pytest
 import oracle
 from conftest import assert_close
 from enargeia_amd import kernels as K
-from test_gpu_prefill import model_tol, run_prefill
+from test_gpu_prefill import model_tol, run_prefill, run_swiglu
 from test_gpu_prefill_rows import device_with
 
 pytestmark = pytest.mark.gpu
@@ -21,8 +22,8 @@ def weights(n, k, bits, fmt, bs):
 
 
 @pytest.mark.parametrize("m,n,k,bits,fmt,bs", [
-    (1, 64, 32, 4, "sym", 32), (33, 100, 160, 4, "sym", 32), (31, 70, 192, 8, "ref", 64),     # 32 x 64
-    (300, 2200, 160, 4, "sym", 32), (290, 2250, 192, 8, "sym", 32),                           # 64 x 64
+    (1, 64, 32, 4, "sym", 32), (33, 100, 160, 4, "sym", 32), (31, 70, 192, 8, "ref", 64),     # 32 x 64 fine
+    (300, 2200, 160, 4, "sym", 32), (290, 2250, 192, 8, "sym", 32),                           # 64 x 64 fine
     (330, 3300, 160, 4, "ref", 32),                                                           # 64 x 128
     (300, 3400, 2080, 4, "sym", 32),                                                          # 64 x 128 deep
     (450, 4600, 96, 4, "sym", 32), (450, 4600, 192, 8, "ref", 64),                            # 64 x 256
@@ -40,8 +41,29 @@ def test_tile_edges_match_the_bf16_model(device, m, n, k, bits, fmt, bs):
     assert_close(got, model, *model_tol(model), label=f"{m}x{n}x{k} int{bits} {fmt} {bs}")
 
 
-TILES = {"32 x 64 fine": "64,1,1,4", "32 x 64": "128,1,1,4", "64 x 64": "128,2,1,4", "64 x 128": "64,2,2,2",
-         "64 x 128 deep": "128,2,2,4", "64 x 256": "128,2,4,1", "128 x 128": "128,4,2,2", "128 x 256": "128,4,4,1"}
+TILES = {"32 x 64 fine": "64,1,1,4", "64 x 64 fine": "64,2,1,4", "32 x 64": "128,1,1,4", "64 x 64": "128,2,1,4",
+         "64 x 128": "64,2,2,2", "64 x 128 long": "128,2,2,2", "64 x 128 deep": "128,2,2,4", "64 x 256": "128,2,4,1",
+         "128 x 128": "128,4,2,2", "128 x 256": "128,4,4,1"}
+
+
+@pytest.mark.parametrize("m,n,k,tile", [
+    (70, 200, 736, "32 x 64 fine"), (300, 2200, 736, "64 x 64 fine"), (33, 100, 1440, "32 x 64"),
+    (290, 1670, 1440, "64 x 64"), (330, 3300, 736, "64 x 128"), (600, 4600, 416, "64 x 256"),
+    (1030, 4170, 416, "128 x 256"), (200, 2300, 2112, "32 x 64"), (20, 5000, 4512, "32 x 64"),
+    (300, 2200, 2080, "64 x 64"), (100, 1400, 8224, "64 x 128 long"), (300, 3400, 2080, "64 x 128 deep"),
+    (520, 3910, 2080, "128 x 128")])
+def test_the_library_chooses(device, m, n, k, tile):
+    """The library's own choice at a shape of each line of its rule: a launch sums in the order of its
+    chunks and K groups, so it equals the tile's forced launch to the bit (K is long enough that the
+    other orders differ)."""
+    x = oracle.normal_floats(m * k, m, 1.0)
+    q = weights(n, k, 4, "sym", 32)
+    forced = device_with(TILES[tile])
+    try:
+        np.testing.assert_array_equal(run_prefill(device, x, q, None, m).view(np.uint32),
+                                      run_prefill(forced, x, q, None, m).view(np.uint32))
+    finally:
+        forced.close()
 
 
 @pytest.mark.parametrize("tile", list(TILES))
@@ -62,6 +84,32 @@ def test_cut_runs_of_columns(tile, n):
             assert not got[m * n:].any()
     finally:
         dev.close()
+
+
+@pytest.mark.parametrize("m,n,k,tile", [
+    *((130, 300, 416, TILES[t]) for t in TILES if t not in ("64 x 128 long", "64 x 128 deep", "128 x 128")),
+    (600, 4864, 160, None), (1030, 4164, 160, None)])
+def test_swiglu_tiles(device, m, n, k, tile):
+    """The paired launch with each tile that has one, and at rows for which the library takes the
+    64 x 256 and 128 x 256 ones, against gate | up and silu_mul_rows to the bit."""
+    x = oracle.normal_floats(m * k, 11, 1.0)
+    gate, up = (oracle.quantize_sym(oracle.normal_floats(n * k, s, 0.05), n, k, 4, 32) for s in (12, 13))
+    paired = device_with(tile) if tile else device
+    os.environ["EG_PREFILL_PAIR"] = "0"
+    try:
+        apart = device_with(tile or "")
+    finally:
+        del os.environ["EG_PREFILL_PAIR"]
+    try:
+        got, want = (run_swiglu(d, x, gate, up, m) for d in (paired, apart))
+        np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+        g, u = (oracle.linear_q_bf16_fast(x, w, None, m).astype(np.float64) for w in (gate, up))
+        ref = g / (1 + np.exp(-g)) * u
+        assert np.linalg.norm(got - ref) <= 1e-4 * np.linalg.norm(ref)  # f32 sums
+    finally:
+        apart.close()
+        if tile:
+            paired.close()
 
 
 @pytest.mark.parametrize("m,n,k", [(70, 96, 96), (450, 4600, 96), (1030, 4170, 96)])
