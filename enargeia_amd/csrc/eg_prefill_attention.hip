@@ -106,6 +106,7 @@ struct Splits {
   float* o;          // NULL: no split, out written directly
   uint32_t keys;     // keys per split (a multiple of kK)
   uint32_t count;    // splits (grid.z)
+  uint32_t first;    // the launch's first query block (see over_blocks)
 };
 
 constexpr float kLog2e = 1.44269504088896340736f;
@@ -151,7 +152,7 @@ __global__ __launch_bounds__(256, 5) void attention_kernel(const float* __restri
   const uint32_t h = blockIdx.x, kv = h / (d.heads / d.kv_heads);
   // the last query blocks (the longest causal walks) first, so they do not start last; heads vary
   // fastest, which deals every length of walk to each XCD
-  const uint32_t q0 = (gridDim.y - 1 - blockIdx.y) * kQ;
+  const uint32_t q0 = (sp.first + gridDim.y - 1 - blockIdx.y) * kQ;
   const uint32_t query = q0 + wave * 16 + lr;  // this lane's query (its column of S^T and O^T)
 
   // Q^T fragments (B operand of S^T = K Q^T): query lr, d 32 ks + 8 lg .. +8.
@@ -327,7 +328,8 @@ __global__ __launch_bounds__(256, 5) void attention_kernel(const float* __restri
 // a tile's values are summed by themselves before they are added. MFMA-bound: 128 of 32 cycles per wave and
 // tile. Against a workgroup per query row with f32 FMAs: 256 queries at keys up to 2048, 14 / 2 heads,
 // 208.7 -> 35.3 us on MI355X (RoPE, append and combine included).
-constexpr uint32_t kF32Group = 8;  // query heads per kv head
+constexpr uint32_t kF32Group = 8;  // query heads per kv head that eg_attention_prefill_f32 takes (a limit of the
+                                   // entry point, not of this kernel)
 constexpr uint32_t kF32Tile = kK * kD * 4;  // bytes of a K (or V) tile
 
 // SHORT: a tile that holds no more than 16 keys takes the products of those alone, for chunks that end
@@ -343,7 +345,7 @@ __global__ __launch_bounds__(256, 2) void attention_f32_kernel(const float* __re
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t lr = lane & 15u, lg = lane >> 4;
   const uint32_t h = blockIdx.x, kv = h / (d.heads / d.kv_heads);
-  const uint32_t q0 = (gridDim.y - 1 - blockIdx.y) * kQ;  // the longest causal walks first
+  const uint32_t q0 = (sp.first + gridDim.y - 1 - blockIdx.y) * kQ;  // the longest causal walks first
   const uint32_t query = q0 + wave * 16 + lr;
 
   float qb[16];
@@ -623,7 +625,7 @@ int eg::check_attention_prefill(eg_context* ctx, const char* op, const eg_attent
   if ((uint64_t)d.max_context * d.kv_heads * d.head_dim * 2 >= (1ull << 31))
     return eg::fail(ctx, EG_ERR_RANGE, "%s: a cache of %u positions x %u kv heads exceeds 2 GiB", op, d.max_context,
                     d.kv_heads);
-  if (d.heads > 65535 || (d.queries + kQ - 1) / kQ > 0x7FFFFFFFu)
+  if (d.heads > 65535)
     return eg::fail(ctx, EG_ERR_RANGE, "%s: %u heads over the grid limit", op, d.heads);
   return EG_OK;
 }
@@ -650,13 +652,25 @@ Splits splits_for(eg_context* ctx, const eg_attention_prefill_dims& d, uint32_t 
   }
   const uint64_t rows = (uint64_t)d.queries * d.heads;
   while (splits > 1 && (uint64_t)splits * rows * (kD + 2) * 4 > eg::kPartialsBytes) splits--;
-  Splits sp{nullptr, 0, 1};
+  Splits sp{nullptr, 0, 1, 0};
   if (splits > 1) {
     sp.keys = ((tiles + splits - 1) / splits) * kK;
     sp.count = (d.keys + sp.keys - 1) / sp.keys;
     sp.o = reinterpret_cast<float*>(eg::partials(ctx));
   }
   return sp;
+}
+
+// Runs launch(grid, sp) over a chunk's query blocks: one launch, as a grid's y takes 65535, or several, the
+// longest walks first.
+template <class F>
+void over_blocks(const eg_attention_prefill_dims& d, Splits sp, F launch) {
+  constexpr uint32_t kMost = 65535;
+  const uint32_t blocks = (d.queries - 1) / kQ + 1;
+  for (uint32_t end = blocks; end > 0; end = sp.first) {
+    sp.first = end > kMost ? end - kMost : 0;
+    launch(dim3(d.heads, end - sp.first, sp.count), sp);
+  }
 }
 
 }  // namespace
@@ -671,8 +685,10 @@ int eg::attention_prefill_run(eg_context* ctx, const float* q_rope, const uint16
   if (d.queries == 0) return EG_OK;
   const uint64_t rows = (uint64_t)d.queries * d.heads;
   const Splits sp = splits_for(ctx, d);
-  hipLaunchKernelGGL(attention_kernel, dim3(d.heads, (d.queries + kQ - 1) / kQ, sp.count), dim3(256), 0, ctx->stream,
-                     q_rope, k_cache, v_cache, out, d, sp, out_bf16 ? 1u : 0u);
+  over_blocks(d, sp, [&](dim3 grid, const Splits& part) {
+    hipLaunchKernelGGL(attention_kernel, grid, dim3(256), 0, ctx->stream, q_rope, k_cache, v_cache, out, d, part,
+                       out_bf16 ? 1u : 0u);
+  });
   if (sp.o) {
     const uint64_t total = rows * kD;
     const uint32_t cblocks = (uint32_t)std::min<uint64_t>((total / 4 + 255) / 256, (uint64_t)ctx->cu_count * 8);
@@ -714,18 +730,17 @@ extern "C" int eg_attention_prefill_f32(eg_context* ctx, const float* q, const f
   if (d.heads / d.kv_heads > kF32Group)
     return eg::fail(ctx, EG_ERR_INVALID, "%s: %u query heads per kv head (at most %u)", op, d.heads / d.kv_heads,
                     kF32Group);
-  if (d.kv_heads > 65535) return eg::fail(ctx, EG_ERR_RANGE, "%s: %u kv heads exceed the grid", op, d.kv_heads);
   if ((reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache) |
        reinterpret_cast<uintptr_t>(q_rope)) & 15u)
     return eg::fail(ctx, EG_ERR_INVALID, "%s: the caches and q_rope must be 16-byte aligned", op);
   hipLaunchKernelGGL(rope_append_kernel<float>, dim3(d.queries), dim3(256), 0, ctx->stream, q, k, v, q_rope, k_cache,
                      v_cache, d);
-  const uint32_t blocks = (d.queries + kQ - 1) / kQ;
   const uint64_t rows = (uint64_t)d.queries * d.heads;
   const Splits sp = splits_for(ctx, d, 2);
   const auto kernel = d.keys <= 2u * kK ? attention_f32_kernel<true> : attention_f32_kernel<false>;
-  hipLaunchKernelGGL(kernel, dim3(d.heads, blocks, sp.count), dim3(256), 0, ctx->stream, q_rope, k_cache,
-                     v_cache, out, d, sp);
+  over_blocks(d, sp, [&](dim3 grid, const Splits& part) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, ctx->stream, q_rope, k_cache, v_cache, out, d, part);
+  });
   if (sp.o) {
     const uint32_t cblocks = (uint32_t)std::min<uint64_t>((rows * kD / 4 + 255) / 256, (uint64_t)ctx->cu_count * 8);
     hipLaunchKernelGGL(combine_kernel, dim3(cblocks), dim3(256), 0, ctx->stream, sp.o, out, (uint32_t)rows, sp.count, 0u,
