@@ -4,8 +4,8 @@
 // The prompt's projections are the dense contraction on the path. This file holds the host side:
 // the checks, the choice of a tile for a shape (tile_for) and the launches. The kernel is
 // gemm_kernel (eg_gemm_kernel.hpp), instantiated in eg_gemm_{bf16,f32,norm,pair,rope}.hip.
-// Layouts it does not take (K or the block size not a multiple of 16 or 32 codes, a block size
-// that is not a power of two, unaligned streams) stage both operands element by element with the
+// Layouts it does not take (K not a multiple of 32 codes or the block size of 16, a block size that
+// is not a power of two, unaligned streams) stage both operands element by element with the
 // reference's indexing (element_kernel below).
 #include <algorithm>
 
@@ -521,7 +521,7 @@ int launch_multi(eg_context* ctx, const void* x, uint32_t first, uint32_t m, uin
   KernelFn fn = nullptr;
   if (epi == kRope) fn = pick_rope(encoding, xm, t);
   else if (epi == kPair) fn = pick_pair(encoding, xm, t);
-  else if (xm == kXNorm) fn = pick_store_norm(encoding, 4, t);
+  else if (xm == kXNorm) fn = pick_store_norm(encoding, t);
   else fn = xm == kXBf16 ? pick_store_bf16(encoding, 4, t) : pick_store_f32(encoding, 4, t);
   const int st = launch_tile(ctx, "matmul_q4_prefill", fn, a, t, 1);
   return st != EG_OK ? st : eg::check_launch(ctx, "matmul_q4_prefill");

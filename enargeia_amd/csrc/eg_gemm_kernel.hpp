@@ -620,7 +620,7 @@ struct Tile {
   // launches of few tiles only, which take the small ones
   bool bf16_only() const { return mf * wn * kg >= 16; }
   bool store_only() const { return bk == 128 && wn == 2; }
-  bool folds_norm() const { return wn == 1 || (wn == 2 && bk == 64); }
+  bool folds_norm() const { return wn == 1; }
   // the tile that takes a bf16_only one's f32 rows: its chunks and K groups, half its rows or columns
   Tile f32_form() const { return kg == 4 ? Tile{bk, mf, wn / 2, kg} : Tile{bk, mf / 2, wn, kg}; }
 };
@@ -638,10 +638,10 @@ KernelFn pick_tile(const Tile& t) {
   if (t.bk == B && t.mf == M && t.wn == W && t.kg == G) return gemm_kernel<ENC, BITS, B, M, W, G, XM, EPI>;
   EG_GEMM_CASE(128, 1, 1, 4)
   EG_GEMM_CASE(128, 2, 1, 4)
-  EG_GEMM_CASE(64, 2, 2, 2)
   EG_GEMM_CASE(64, 1, 1, 4)
   EG_GEMM_CASE(64, 2, 1, 4)
   if constexpr (XM != kXNorm) {
+    EG_GEMM_CASE(64, 2, 2, 2)
     EG_GEMM_CASE(128, 2, 4, 1)
     if constexpr (EPI == kStore) {
       EG_GEMM_CASE(128, 2, 2, 2)
@@ -661,7 +661,7 @@ KernelFn pick_tile(const Tile& t) {
 // One translation unit per x mode and epilogue group, so they compile in parallel.
 KernelFn pick_store_bf16(int encoding, int bits, const Tile& t);
 KernelFn pick_store_f32(int encoding, int bits, const Tile& t);
-KernelFn pick_store_norm(int encoding, int bits, const Tile& t);
+KernelFn pick_store_norm(int encoding, const Tile& t);
 KernelFn pick_pair(int encoding, int xm, const Tile& t);
 KernelFn pick_rope(int encoding, int xm, const Tile& t);
 
