@@ -25,7 +25,8 @@ struct eg_context {
   // bf16 rows of a prefill GEMM's f32 x (eg_gemm.hip), eg::kRowsBytes. Not the workspace's other half: in
   // one allocation of 128 MiB the chunk attention's splits took longer to write and merge (1 query at
   // 3227, 16 splits: 17.3 us for 16.5).
-  void* rows = nullptr;
+  uint8_t* rows = nullptr;
+  size_t rows_next = 0;  // where the next call's start
   bool capturing = false;
   // This device's copy of the fixed scratch array of eg_lm_head_argmax_noalloc (resolved by
   // eg::noalloc_scratch_init at creation; shared by every context on the device).

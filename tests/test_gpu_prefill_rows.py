@@ -131,6 +131,30 @@ def test_rows_past_the_buffer():
         dev.close()
 
 
+def test_calls_in_a_row_go_round_the_buffer():
+    """Ten calls of 16 MiB of rows, none waited for: each gives what it gives alone."""
+    m, n, k = 2048, 130, 4096
+    dev = device_with("128,4,2,2,1")
+    calls = [Gemm(dev, m, n, k) for _ in range(10)]
+    try:
+        base = oracle.normal_floats(m * k, 6, 1.0)
+        for i, g in enumerate(calls):
+            g.set_x(np.roll(base, 977 * i))
+        for g in calls:
+            g.encode()
+        got = [g.read() for g in calls]
+        for g, y in zip(calls, got):
+            g.encode()
+            np.testing.assert_array_equal(g.read(), y)
+        for i in (0, 9):
+            model = oracle.linear_q_bf16_fast(np.roll(base, 977 * i)[:40 * k], calls[i].q, None, 40)
+            assert_close(got[i].view(np.float32)[:40 * n], model, *model_tol(model), label=f"call {i}")
+    finally:
+        for g in calls:
+            g.release()
+        dev.close()
+
+
 def test_a_call_allocates_nothing():
     """The free device memory is the same before and after a context's first wide call."""
     lib = _lib.load()
