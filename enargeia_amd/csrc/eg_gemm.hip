@@ -222,7 +222,7 @@ uint64_t tile_count(const Tile& t, uint32_t m, uint64_t cols) {
 //    256 x 4864 x  896      13.0   14.3        13.5   17.6    11.7    16.4     24.2   (608 | 304 | 152)
 //    256 x 9728 x  896      19.1   21.8        19.3   25.8    17.1    17.1     25.0   (1216 | 608 | 304 | 152)
 //   2048 x 1152 x  896, q|k|v (RoPE)
-//                           23.2   25.0        23.7   27.4    23.8    22.1     29.5   (1152 | 576 | 288 | 160)
+//                           23.5   24.7        23.6   26.6    23.5    22.0     29.7   (1152 | 576 | 288 | 160)
 //    200 x 8960 x 1536      26.5   24.6        27.3   31.1    28.0    23.2     35.8   (980 | 560 | 280 | 140)
 //    512 x 9728 x  896         -      -        29.5   42.7    25.7    26.1     27.8   (2432 | 1216 | 608 | 304)
 //   2048 x 9728 x  896, gate|up (bf16 rows): 64x256 64, 128x256 58
@@ -245,7 +245,7 @@ uint64_t tile_count(const Tile& t, uint32_t m, uint64_t cols) {
 //   2048 x 4096 x 11008 -         420       276          300          221       207
 //
 // RoPE's epilogue (angles, rotation, f16 rows) grows with a tile's rows: 32 up to two workgroups per CU
-// (q|k|v of 600 rows, fine: 11.6 us; 64 x 64, not fine: 13.5). Blocks of 16 codes need the 64-deep chunks.
+// (q|k|v of 600 rows, fine: 11.6 us; 64 x 64, not fine: 13.3). Blocks of 16 codes need the 64-deep chunks.
 Tile tile_for(const eg_context* ctx, uint32_t m, uint64_t cols, uint32_t k, uint32_t bs, uint64_t launch_cols,
               int epi) {
   if (ctx->gemm_tile[0]) {

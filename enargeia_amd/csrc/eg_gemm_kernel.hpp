@@ -420,12 +420,19 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_kernel(Args a) {
   }
 
   // ---- epilogue: unit (i, p) = row fragment i with columns 8 p + 4 g .. +4 of both column fragments --
-  // kRope: cos and sin of unit (i, p)'s four pairs, which the callers read ahead of the sums
-  struct Angles {
+  // kRope: cos and sin of unit (i, p)'s four pairs and their biases, which the callers read ahead of the
+  // sums (read where they are added, the biases took a round trip to memory per unit: q|k|v of 2048 rows,
+  // its norm's launch included, 28.5 us for 23.2)
+  struct Ahead {
     double2 cs[EPI == kRope ? 4 : 1];
+    f32x4 bias[2];
   };
-  auto angles_of = [&](uint32_t i, uint32_t p, Angles& c) {
-    if (EPI != kRope || si == 2) return;
+  auto read_ahead = [&](uint32_t i, uint32_t p, Ahead& c) {
+    if (EPI != kRope) return;
+    const float* b = w0.bias ? w0.bias + n0 + 8u * p + 4u * g : nullptr;
+#pragma unroll
+    for (int h = 0; h < 2; h++) c.bias[h] = b ? (f32x4)*reinterpret_cast<const f32x4u*>(b + 32 * h) : f32x4{0.f, 0.f, 0.f, 0.f};
+    if (si == 2) return;
     const uint32_t row = min(m0 + 32u * i + lr, a.m - 1);
 #pragma unroll
     for (int e = 0; e < 4; e++) c.cs[EPI == kRope ? e : 0] = a.rope[(size_t)(a.rope_pos0 + row) * 32u + 8u * p + 4u * g + e];
@@ -457,7 +464,7 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_kernel(Args a) {
     for (int e = 0; e < 4; e++) v[e] = v[e] + (w0.bias ? w0.bias[col + e] : 0.f) + res[e];
     *reinterpret_cast<f32x4u*>(w0.out + o) = v;
   };
-  auto finish = [&](uint32_t i, uint32_t p, f32x4 lo, f32x4 hi, const Angles& an) {
+  auto finish = [&](uint32_t i, uint32_t p, f32x4 lo, f32x4 hi, const Ahead& ahead) {
     const uint32_t r = 32u * i + lr, row = m0 + r;
     if (!active || row >= a.m) return;
     if (XM == kXNorm) {
@@ -493,10 +500,10 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_kernel(Args a) {
       float x[4], y[4];
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        x[e] = lo[e] + (w0.bias ? w0.bias[n0 + c + e] : 0.f) + 0.f;
-        y[e] = hi[e] + (w0.bias ? w0.bias[n0 + c + 32u + e] : 0.f) + 0.f;
+        x[e] = lo[e] + ahead.bias[0][e] + 0.f;
+        y[e] = hi[e] + ahead.bias[1][e] + 0.f;
         if (si < 2) {
-          const float2 rr = egd::rotate(x[e], y[e], an.cs[EPI == kRope ? e : 0]);
+          const float2 rr = egd::rotate(x[e], y[e], ahead.cs[EPI == kRope ? e : 0]);
           x[e] = rr.x;
           y[e] = rr.y;
         }
@@ -536,9 +543,9 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_kernel(Args a) {
     for (int i = 0; i < MF; i++)
 #pragma unroll
       for (int p = 0; p < 4; p++) {
-        Angles an;
-        angles_of(i, p, an);
-        finish(i, p, run(acc[0][i], p), run(acc[1][i], p), an);
+        Ahead ahead;
+        read_ahead(i, p, ahead);
+        finish(i, p, run(acc[0][i], p), run(acc[1][i], p), ahead);
         __builtin_amdgcn_sched_barrier(0);  // one unit at a time: together they spill
       }
   } else if constexpr (EPI == kStore) {
@@ -591,9 +598,9 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_kernel(Args a) {
 #pragma unroll
       for (int u = 0; u < 4 * MF; u++) sums[at(group, f, u)] = run(acc[f][u / 4], u % 4);
     static_assert(4 * MF % KG == 0, "the groups share the units");
-    Angles an[4 * MF / KG];
+    Ahead ahead[4 * MF / KG];
 #pragma unroll
-    for (uint32_t v = 0; v < 4u * MF / KG; v++) angles_of((group + v * KG) / 4, (group + v * KG) % 4, an[v]);
+    for (uint32_t v = 0; v < 4u * MF / KG; v++) read_ahead((group + v * KG) / 4, (group + v * KG) % 4, ahead[v]);
     __syncthreads();
 #pragma unroll
     for (uint32_t v = 0; v < 4u * MF / KG; v++) {
@@ -604,7 +611,7 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_kernel(Args a) {
         lo += sums[at(q, 0, u)];
         hi += sums[at(q, 1, u)];
       }
-      finish(u / 4, u % 4, lo, hi, an[v]);
+      finish(u / 4, u % 4, lo, hi, ahead[v]);
     }
   }
 }
