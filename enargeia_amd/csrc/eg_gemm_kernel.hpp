@@ -453,7 +453,13 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_kernel(Args a) {
     const size_t o = (size_t)row * w0.out_stride + col + w0.out_offset;
     w0.out[o] = v + (w0.bias ? w0.bias[col] : 0.f) + (w0.residual ? w0.residual[o] : 0.f);
   };
-  auto store4 = [&](uint32_t row, uint32_t col, f32x4 v) {
+  // (their biases, the same for every row, are read once, ahead of the sums: read at each store they took
+  // 256 x 4864 x 896 1.0 us)
+  auto bias4 = [&](uint32_t col) {
+    return !a.partials && w0.bias && active && col + 4 <= w0.n ? (f32x4)*reinterpret_cast<const f32x4u*>(w0.bias + col)
+                                                               : f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  auto store4 = [&](uint32_t row, uint32_t col, f32x4 v, f32x4 bias) {
     if (a.partials) {
       *reinterpret_cast<f32x4u*>(a.partials + ((size_t)blockIdx.y * a.m + row) * w0.n + col) = v;
       return;
@@ -461,7 +467,7 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_kernel(Args a) {
     const size_t o = (size_t)row * w0.out_stride + col + w0.out_offset;
     const f32x4 res = w0.residual ? (f32x4)*reinterpret_cast<const f32x4u*>(w0.residual + o) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int e = 0; e < 4; e++) v[e] = v[e] + (w0.bias ? w0.bias[col + e] : 0.f) + res[e];
+    for (int e = 0; e < 4; e++) v[e] = v[e] + bias[e] + res[e];
     *reinterpret_cast<f32x4u*>(w0.out + o) = v;
   };
   auto finish = [&](uint32_t i, uint32_t p, f32x4 lo, f32x4 hi, const Ahead& ahead) {
@@ -528,7 +534,7 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_kernel(Args a) {
       const uint32_t col = n0 + 8u * p + 32u * h + 4u * g;
       const f32x4 v = h ? hi : lo;
       if (col + 4 <= w0.n) {
-        store4(row, col, v);
+        store4(row, col, v, ahead.bias[h]);
       } else {
 #pragma unroll
         for (int e = 0; e < 4; e++)
@@ -539,12 +545,23 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_kernel(Args a) {
 
   auto run = [](const f32x16& v, int p) { return f32x4{v[4 * p], v[4 * p + 1], v[4 * p + 2], v[4 * p + 3]}; };
   if constexpr (KG == 1) {
+    f32x4 bias[EPI == kStore ? 4 : 1][2];
+    if (EPI == kStore) {
+#pragma unroll
+      for (int p = 0; p < 4; p++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) bias[EPI == kStore ? p : 0][h] = bias4(n0 + 8u * p + 32u * h + 4u * g);
+    }
 #pragma unroll
     for (int i = 0; i < MF; i++)
 #pragma unroll
       for (int p = 0; p < 4; p++) {
         Ahead ahead;
         read_ahead(i, p, ahead);
+        if (EPI == kStore) {
+          ahead.bias[0] = bias[EPI == kStore ? p : 0][0];
+          ahead.bias[1] = bias[EPI == kStore ? p : 0][1];
+        }
         finish(i, p, run(acc[0][i], p), run(acc[1][i], p), ahead);
         __builtin_amdgcn_sched_barrier(0);  // one unit at a time: together they spill
       }
@@ -562,9 +579,10 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_kernel(Args a) {
     for (int f = 0; f < 2; f++)
 #pragma unroll
       for (int u = 0; u < 4 * MF; u++) sums[at(group, f, u, lane)] = run(acc[f][u / 4], u % 4);
+    const uint32_t c = lane & 15u, f = c >> 3, p = (c >> 1) & 3u;
+    const f32x4 bias = bias4(n0 + 4u * c);
     __syncthreads();
     if (!active) return;
-    const uint32_t c = lane & 15u, f = c >> 3, p = (c >> 1) & 3u;
 #pragma unroll
     for (uint32_t v = 0; v < 8u * MF / KG; v++) {
       const uint32_t r = (group + v * KG) * 4u + (lane >> 4), u = (r >> 5) * 4u + p, l = (r & 31u) + 32u * (c & 1u);
@@ -573,7 +591,7 @@ __global__ __launch_bounds__(64 * WN * KG, 2) void gemm_kernel(Args a) {
       for (int q = 1; q < KG; q++) x += sums[at(q, f, u, l)];
       if (m0 + r >= a.m || n0 + 4u * c + 4u > w0.n) continue;
       if (XM == kXNorm) x *= inv_rms(r);
-      store4(m0 + r, n0 + 4u * c, x);
+      store4(m0 + r, n0 + 4u * c, x, bias);
     }
     const uint32_t cut = w0.n & ~3u;  // the cut run's first column
     if (n0 + kCols <= cut || cut == w0.n) return;
