@@ -208,10 +208,10 @@ uint64_t tile_count(const Tile& t, uint32_t m, uint64_t cols) {
 // of these workgroups costs more than larger tiles), and the largest where none does: large tiles spread
 // the dequantization over more rows, small ones fill the device and, with four groups of waves on alternate
 // chunks of K, shorten the serial chain. The small ones take 64-deep chunks ("fine") up to K = 768 and where
-// those leave fewer idle steps to the groups (K of 1025 to 1280), and at 769 to 896, where both leave
-// the same, from half a workgroup per CU on (a gate|up pair is then twice that, and its launches fold the
-// norm: 64 x 4864 x 896 as a pair 10.4 us fine, 11.3 else). Measured on MI355X (us; f32 rows, int4 sym;
-// workgroups of 32x64 | 64x64 | 64x128 | 64x256):
+// those leave fewer idle steps to the groups (K of 1025 to 1280); at 769 to 896, where both leave the
+// same, where a launch or a pair of it takes 64 rows (64 x 4864 x 896 as a pair 10.2 us fine, 11.9 else; 70
+// rows, 32 at a time, of the reference format 10.2 fine, 9.7 else). Measured on MI355X (us; f32 rows, int4
+// sym; workgroups of 32x64 | 64x64 | 64x128 | 64x256):
 //                     32x64 fine  32x64  64x64 fine  64x64  64x128  64x256  128x256
 //     64 x 1024 x  320       5.1    5.3         6.7    7.3     7.9    10.6     13.5   (32)
 //    128 x 4864 x  640       8.3    9.6         8.1    9.3     9.8    13.4     20.8   (304 | 152)
@@ -266,7 +266,8 @@ Tile tile_for(const eg_context* ctx, uint32_t m, uint64_t cols, uint32_t k, uint
   const uint64_t n = count(kTile32x64);
   if (bs < 32) return fits(kTile64x64Fine) ? rows(kTile32x64Fine, kTile64x64Fine) : kTile64x128;
   if (k < 2048) {
-    const bool fine = k <= 768 || (k <= 896 && n > cus / 2) || (k > 1024 && k <= 1280);
+    const bool fine = k <= 768 || (k > 1024 && k <= 1280) ||
+                      (k <= 896 && (n > cus || (n > cus / 2 && count(kTile64x64) <= cus / 2)));
     if (fits(kTile64x64) || (m <= 32 && n <= 2 * cus))
       return fine ? rows(kTile32x64Fine, kTile64x64Fine) : rows(kTile32x64, kTile64x64);
     if (fits(kTile64x128)) return kTile64x128;
