@@ -954,7 +954,7 @@ def prefill_numbers(dev, ev, stream, args) -> dict:
         pairs = H * sum(begin + i + 1 for i in range(M))
         tf = 4.0 * D * pairs / (us * 1e-6) / 1e12
         res[f"attention_m{M}_begin{begin}"] = {"us": round(us, 2), "tflops": round(tf, 3)}
-    # the same chunk over an f32 cache (eg_attention_prefill_f32: exact rows, f32 FMAs)
+    # the same chunk over an f32 cache (eg_attention_prefill_f32: exact rows, f32 MFMAs)
     caches32 = [dev.upload(rng.standard_normal(CTX * KVH * D, dtype=np.float32)) for _ in range(2)]
     keep += caches32
     for begin in (0, CTX - M):

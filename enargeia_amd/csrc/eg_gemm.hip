@@ -181,8 +181,9 @@ void to_bf16(eg_context* ctx, const float* x, size_t n, void* out) {
 }
 
 // How many rows of k f32 values the context's buffer takes as bf16 at once, in whole tiles; 0: none, and
-// the launch stages f32 rows. The buffer is used on the context's own stream alone and outside captures: every use is then ordered after the one before it, whatever other streams and
-// replayed graphs do beside it.
+// the launch stages f32 rows. The buffer is used on the context's own stream alone and outside captures:
+// every use is then ordered after the one before it, whatever other streams and replayed graphs do beside
+// it.
 uint32_t rows_at_once(const eg_context* ctx, uint32_t k, const Tile& t) {
   if (ctx->stream != ctx->own_stream || ctx->capturing) return 0;
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;

@@ -14,8 +14,8 @@
 //
 // The k order. Chunk c covers k in [c BK, (c + 1) BK); lane group g = lane / 32 owns k = g BK / 2 +
 // [0, BK / 2) of it, and step s multiplies the groups' 8 k at offset 8 s. x is read from LDS in
-// the same order, so any order gives the whole sum; launches of one shape class use one order, and
-// with it the same bits whatever is folded into their epilogues.
+// the same order, so any order gives the whole sum; it follows from BK, KG and the K splits, which
+// tile_for chooses by one matrix's shape: the same bits whatever a launch folds into its epilogue.
 //
 // The products are formed transposed (W rows as the MFMA's A operand, x rows as B): lane l then
 // holds, for row m = l % 32 of x, runs of four consecutive columns of W - one 16-byte store each,

@@ -59,8 +59,7 @@ struct eg_context {
   bool prefill_rope = true;
   // the prompt chain's GEMM inputs produced as bf16 rows where the GEMM stages them (false: f32)
   bool prefill_xb16 = true;
-  // prefill GEMM tiles mapped so each XCD runs whole row tiles where that applies (false: the
-  // grid's own order)
+  // prefill GEMM tiles dealt to the XCDs in column- or row-major runs (false: the grid's own order)
   bool prefill_xcd = true;
   uint32_t attention_split_tiles = 8;
   uint32_t attention_split_fill = 1;

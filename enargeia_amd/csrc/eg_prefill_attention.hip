@@ -325,9 +325,10 @@ __global__ __launch_bounds__(256, 5) void attention_kernel(const float* __restri
 //   blocks, and a lane's o[0..3][e] are the four consecutive d = 16 g + 4 e .. +4.
 // K and V rows go from memory to LDS directly, the next tile's while this one is multiplied; K's 16-byte
 // slots are swizzled by the row. Sums stay short for their error's sake: a score is two chains of 32 products,
-// a tile's values are summed by themselves before they are added. MFMA-bound: 128 of 32 cycles per wave and
-// tile. Against a workgroup per query row with f32 FMAs: 256 queries at keys up to 2048, 14 / 2 heads,
-// 208.7 -> 35.3 us on MI355X (RoPE, append and combine included).
+// a tile's values are summed by themselves before they are added. A wave and tile take 128
+// MFMAs of 32 cycles: 46% of the SIMDs' cycles (256 queries at 1792, 14 / 2 heads: two workgroups on three
+// quarters of the CUs), vector instructions 24%, LDS conflicts (K's operand) 3%. Against a workgroup per query
+// row with f32 FMAs the same call went from 208.8 to 35.1 us on MI355X (RoPE, append and combine included).
 constexpr uint32_t kF32Group = 8;  // query heads per kv head that eg_attention_prefill_f32 takes (a limit of the
                                    // entry point, not of this kernel)
 constexpr uint32_t kF32Tile = kK * kD * 4;  // bytes of a K (or V) tile

@@ -214,10 +214,9 @@ def test_prefill_swiglu_pair(device, unpaired, m, n, k, sym):
 
 @pytest.mark.parametrize("m,n,k", [(512, 896, 896), (1024, 896, 4864), (1024, 1152, 896)])
 def test_prefill_row_tiles_per_xcd(device, m, n, k):
-    # A multiple of 8 row tiles and a column-tile count that is not: the launch maps whole row
-    # tiles to each XCD (workgroup L of the grid runs tile (L / 8 % columns, L % 8 + 8 * (L / 8 /
-    # columns))), every tile exactly once - against the bf16 model like any other shape. The
-    # K = 4864 case splits K and keeps the grid's own order.
+    # Many row tiles and a column-tile count that is no multiple of 8: each XCD takes a run of
+    # the tiles, column- or row-major, every tile exactly once - against the bf16 model like any
+    # other shape.
     x, q = config3(m, n, k, 0x5EED ^ (m + n + k))
     got = run_prefill(device, x, q, None, m)
     model = oracle.linear_q_bf16_fast(x, q, None, m)

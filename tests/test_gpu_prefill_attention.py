@@ -87,8 +87,8 @@ def test_prefill_attention_matches_oracle(device, begin, n):
 def test_prefill_attention_f32_cache_matches_oracle(device, begin, n, heads, kv_heads):
     """eg_attention_prefill_f32: q_rope as the f16 variant's; the appended rows RoPE(k) (one ulp
     for the double-precision angle) and v exactly, f32; the output over the exact rows within
-    the decode attention's f32 bar (1e-5 x rms + 2e-5 relative: f32 FMAs and one exp per score
-    against float64)."""
+    the decode attention's f32 bar (1e-5 x rms + 2e-5 relative: f32 products and sums
+    and one exp per score against float64)."""
     print(f"prefill attention f32 begin {begin} queries {n} heads {heads}/{kv_heads}", flush=True)
     rng = np.random.default_rng(2000 + begin + n)
     q = rng.standard_normal((n, heads * D), dtype=np.float32)

@@ -289,8 +289,8 @@ def test_prefill_fused_launches_match_unfused_bit_exactly(device, switch, chunk)
 
 
 def test_prefill_row_tiles_per_xcd_bit_exact(device):
-    """A 512-token prompt (8 row tiles: the o, down and q|k|v launches map whole row tiles to
-    each XCD) against the grid's own order (EG_PREFILL_XCD=0), logits and caches to the bit."""
+    """A 512-token prompt (its GEMM launches deal each XCD a run of their tiles) against the
+    grid's own order (EG_PREFILL_XCD=0), logits and caches to the bit."""
     import os
     from enargeia_amd import kernels as K
     os.environ["EG_PREFILL_XCD"] = "0"
